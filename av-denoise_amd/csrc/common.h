@@ -28,10 +28,9 @@ struct NlmWindow {
     float offset;        // pair: the flat noise offset
     int step, blocks_x, blocks_y;
 };
-// `variant` picks the rows each wave walks (0: 16, 1: 8, 2: 4); every variant gives bit-identical
+// `variant` picks the columns each lane walks (0: 8, 1: 4, 2: 2); every variant gives bit-identical
 // sums, so the tuner may choose any (kNlmVariants of them).
 constexpr int kNlmVariants = 3;
-int nlm_variant_rows(int variant);
 hipError_t launch_nlm_single(const NlmWindow &w, const float *frame, const float *lut, float *accum, float *wsum,
                              float *maxw, hipStream_t s, int variant = 0);
 hipError_t launch_nlm_pair(const NlmWindow &w, const float *centre, const float *fwd, const float *bwd,
@@ -50,7 +49,7 @@ struct NlmFrames {
 };
 // The batched form: every pair, the single window and the finish of one frame in one launch, the
 // window sums kept on chip; bit-identical to launch_nlm_pair (each pair) + launch_nlm_single +
-// launch_nlm_finish on zeroed accumulators.  `variant` picks 8 (0) or 4 (1) rows per wave.
+// launch_nlm_finish on zeroed accumulators.  `variant` picks 8 (0) or 4 (1) columns per lane.
 constexpr int kNlmBatchedVariants = 2;
 hipError_t launch_nlm_window(const NlmWindow &w, const NlmFrames &f, const float *centre, const float *lut,
                              float self_weight, float *out, hipStream_t s, int variant = 0);

@@ -9,18 +9,28 @@
 // sum(w * y), sum(w) and max(w) in registers, added to the accumulators once.  nlm_finish
 // (accumulate.rs:54-101) then blends in the centre with self_weight * max_w.
 //
-// MI355X layout.  A wavefront owns 64 adjacent distance columns: lane l holds the distance of
-// image column X0 - P + l, and after the horizontal box sum lane l (l >= 2P) owns output column
-// X0 - 2P + l.  The horizontal sum is a chain of 2P DPP wave_shr:1 adds (each a single v_add_f32
-// with a DPP source), so it needs no LDS and no barrier.  Each lane walks ROWS output rows of its
-// column: the centre values of its ROWS + 2P distance rows stay in registers for the whole
-// window, and the vertical box sum adds 2P+1 of the row sums kept in registers.  ROWS (16, 8 or 4)
-// trades the 2P halo rows each wave recomputes against the number of waves a small frame spreads
-// over; every choice gives bit-identical sums, and the tuner picks one per window shape.  The neighbour
-// frame(s) of the workgroup are staged once in LDS with their (P+s) halo, so the offset loop runs
-// with no barrier at all.  On planes up to 2^20 pixels each row group's offsets are split over SPLIT
-// waves whose sums then add in LDS in part order, so small frames still fill the chip.
+// MI355X layout.  The lanes of a wavefront are 64 adjacent distance rows and each lane walks COLS
+// output columns, so the horizontal box sum runs in the lane's registers (2P fused multiply-adds that
+// also apply the channel scale) and the vertical one is a chain of 2P v_add_f32 whose shifted operand
+// is a DPP wave_shr:1 (lane l then holds the sum of rows l - 2P .. l, added top to bottom; lanes from
+// 2P on own an output row).  Lanes on columns instead, the sums the other way round, cost two
+// instructions per horizontal step, since no fused multiply-add takes a DPP operand as its addend, and
+// recompute a 2P-row halo of them per COLS rows.  The neighbour frame(s) of the workgroup are staged
+// in LDS with their (P + s) halo at an odd row pitch (64 lanes on 64 rows then hit distinct banks, and
+// a lane's columns are immediate offsets), so the offset loop runs with no barrier.  COLS (8, 4 or 2)
+// trades the 2P halo columns each lane recomputes (differences only) against the number of waves a
+// small frame spreads over; every choice gives bit-identical sums, and the tuner picks one per window
+// shape.  On planes up to 2^20 pixels each tile's offsets are split over SPLIT waves whose sums add in
+// part order.  The sums leave through LDS, so global accumulators are read and written along rows.
+// Bound by vector instruction issue: per pixel and offset about 2 (1 + 2P / COLS) for the differences,
+// 4P + 1 for the box sums and 10 for the weight (v_exp_f32 issues over four cycles) and the sums.
+// Against lanes on columns (one pair or window of one frame, same sums): 640x360 P 2 S 7 81 -> 42 us,
+// 1920x1080 P 3 S 4 pair 541 -> 266 us, P 4 S 2 pair with confidence 276 -> 120 us, two-channel 960x540
+// P 3 S 4 pair 300 -> 113 us; the first runs at 85 % of its instruction issue bound (36 us at 240
+// workgroups on 256 CUs).
 // exp is v_exp_f32 (exp2) with log2(e) folded into h2 on the host.
+#include <algorithm>
+
 #include "common.h"
 
 namespace avd {
@@ -30,247 +40,279 @@ namespace {
 constexpr int kMaxP = 8;
 constexpr int kMaxS = 8;
 
+// Lane l reads lane l - 1; lane 0 reads 0.
 __device__ __forceinline__ float wave_shr1(float v)
 {
-    // DPP wave_shr:1: lane l reads lane l-1; lane 0 reads 0.
-    return __builtin_amdgcn_update_dpp(0.0f, v, 0x138, 0xf, 0xf, false);
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x138, 0xf, 0xf, true));
 }
 
 __device__ __forceinline__ int clampi(int v, int hi) { return v < 0 ? 0 : (v > hi ? hi : v); }
 
-// Loads a clamped (rows x cols) window of an interleaved frame into LDS.
-template <int C, int WV>
-__device__ void stage_tile(float *tile, const float *__restrict__ frame, int W, int H, int x0, int y0, int cols,
-                           int rows)
+// Shape of a workgroup: WX waves side by side, COLS output columns each, by SPLIT offset parts; its
+// tile is 64 - 2P output rows high.
+template <int C, int P, int COLS, int WX, int SPLIT>
+struct Shape {
+    static constexpr int kWidth = WX * COLS;         // output columns
+    static constexpr int kRows = 64 - 2 * P;         // output rows
+    static constexpr int kThreads = WX * SPLIT * 64;
+    static constexpr int kDist = COLS + 2 * P;       // distance columns of a lane
+    // Output elements a thread finishes: of the 64 x kWidth grid, element t + k kThreads.
+    static constexpr int kElems = (64 * kWidth + kThreads - 1) / kThreads;
+    // Lanes that stage one tile row: at least its columns at the largest search radius.
+    static constexpr int kStage = kWidth + 2 * P + 2 * kMaxS <= 32 ? 32 : 64;
+    static_assert(kWidth + 2 * P + 2 * kMaxS <= 64, "a tile row is staged by at most 64 lanes");
+};
+
+// Samples between rows of a staged tile: odd, so that lanes on consecutive rows fall on distinct banks.
+__host__ __device__ inline int tile_pitch(int width, int P, int S) { return (width + 2 * P + 2 * S) | 1; }
+
+// Loads the clamped (rows x cols) window of an interleaved frame from (x0, y0) into LDS, LANES lanes
+// to a row and four rows of loads in flight.
+template <int C, int THREADS, int LANES>
+__device__ __forceinline__ void stage_tile(float *tile, const float *__restrict__ frame, int W, int H, int x0, int y0,
+                                           int cols, int rows, int pitch)
 {
-    const int n = cols * rows;
-    for (int i = threadIdx.x; i < n; i += WV * 64) {
-        const int ty = i / cols, tx = i - ty * cols;
-        const int sx = clampi(x0 + tx, W - 1), sy = clampi(y0 + ty, H - 1);
-        const float *src = frame + ((size_t)sy * W + sx) * C;
+    constexpr int kStep = THREADS / LANES, kBatch = 4;
+    const int tx = threadIdx.x % LANES, first = threadIdx.x / LANES;
+    const float *column = frame + (size_t)clampi(x0 + tx, W - 1) * C;
+    for (int r = first; r < rows; r += kStep * kBatch) {
+        float v[kBatch][C];
 #pragma unroll
-        for (int c = 0; c < C; ++c) tile[(size_t)i * C + c] = src[c];
+        for (int u = 0; u < kBatch; ++u) {
+            const float *src = column + (size_t)clampi(y0 + min(r + u * kStep, rows - 1), H - 1) * W * C;
+#pragma unroll
+            for (int c = 0; c < C; ++c) v[u][c] = src[c];
+        }
+#pragma unroll
+        for (int u = 0; u < kBatch; ++u) {
+            const int row = r + u * kStep;
+            if (row < rows && tx < cols) {
+#pragma unroll
+                for (int c = 0; c < C; ++c) tile[((size_t)row * pitch + tx) * C + c] = v[u][c];
+            }
+        }
     }
 }
 
-// The offset loop of one window for this lane's ROWS output rows, into acc / ws / mw (zeroed
-// here): every offset q (q != 0 for a single window) against the staged tile `tf` (the forward
-// frame of a pair, or the frame itself) and, for a pair, `tb` (the backward frame at -q).  `cen`
-// holds the lane's centre column of ROWS + 2P distance rows; `tcols` is the tiles' row pitch.
-template <int C, int P, int ROWS, bool PAIR, bool CONF, int SPLIT>
-__device__ __forceinline__ void window_sums(const NlmWindow &w, const float *tf, const float *tb, int tcols, int wave,
-                                            int lane, int part, const float (&cen)[ROWS + 2 * P][C],
-                                            const float *__restrict__ lut, const float (&conf_fv)[ROWS],
-                                            const float (&conf_bv)[ROWS], float (&acc)[ROWS][C], float (&ws)[ROWS],
-                                            float (&mw)[ROWS])
+// The weights of this lane's COLS output pixels at one offset: the distances of row `nb` (the staged
+// row of this lane at the offset) to `cen`, their (2P+1)^2 box sums and the exponential.  Every
+// operation is spelled out (no contraction): the sums of all launch forms and tile shapes are the same.
+template <int C, int P, int COLS>
+__device__ __forceinline__ void offset_weights(const float *nb, const float (&cen)[COLS + 2 * P][C], float scale,
+                                               float off, float h2l, float (&weight)[COLS])
 {
-    constexpr int DR = ROWS + 2 * P;
-    const int S = w.S;
-    const float scale = (C == 1) ? 3.0f : 1.5f;
+#pragma clang fp contract(off)
+    float sq[COLS + 2 * P];
+#pragma unroll
+    for (int i = 0; i < COLS + 2 * P; ++i) {
+        const float e0 = cen[i][0] - nb[i * C];
+        if constexpr (C == 1) {
+            sq[i] = e0 * e0;
+        } else {
+            const float e1 = cen[i][1] - nb[i * C + 1];
+            sq[i] = fmaf(e0, e0, e1 * e1);
+        }
+    }
+    float h[COLS], d[COLS];
+#pragma unroll
+    for (int j = 0; j < COLS; ++j) {
+        float a = scale * sq[j];
+#pragma unroll
+        for (int k = 1; k <= 2 * P; ++k) a = fmaf(scale, sq[j + k], a);
+        h[j] = a;
+        d[j] = a;
+    }
+    // Step by step over all columns, so that a DPP read never follows the write of its operand at once.
+#pragma unroll
+    for (int k = 0; k < 2 * P; ++k)
+#pragma unroll
+        for (int j = 0; j < COLS; ++j) d[j] = wave_shr1(d[j]) + h[j];
+#pragma unroll
+    for (int j = 0; j < COLS; ++j) weight[j] = __builtin_amdgcn_exp2f(-fmaxf(d[j] - off, 0.0f) * h2l);
+}
+
+// The offset loop of one window for this lane's COLS output pixels, into acc / ws / mw (zeroed here):
+// every offset q (q != 0 for a single window) against the staged tile `tf` (the forward frame of a
+// pair, or the frame itself) and, for a pair, `tb` (the backward frame at -q).  `cen` holds the lane's
+// centre row of COLS + 2P distance columns.
+template <int C, int P, int COLS, bool PAIR, bool CONF, int SPLIT>
+__device__ __forceinline__ void window_sums(const NlmWindow &w, const float *tf, const float *tb, int pitch, int wave,
+                                            int lane, int part, const float (&cen)[COLS + 2 * P][C],
+                                            const float *__restrict__ lut, const float (&conf_fv)[COLS],
+                                            const float (&conf_bv)[COLS], float (&acc)[COLS][C], float (&ws)[COLS],
+                                            float (&mw)[COLS])
+{
+#pragma clang fp contract(off)
+    const int S = w.S, side = 2 * S + 1;
+    float scale = (C == 1) ? 3.0f : 1.5f;
+    asm("" : "+s"(scale));  // in a register: a literal would double the size of every multiply-add
     const float h2l = w.h2_log2e;
 #pragma unroll
-    for (int j = 0; j < ROWS; ++j) {
+    for (int j = 0; j < COLS; ++j) {
 #pragma unroll
         for (int c = 0; c < C; ++c) acc[j][c] = 0.0f;
         ws[j] = 0.0f;
         mw[j] = 0.0f;
     }
-    const int side = 2 * S + 1;
-    // Tile coordinates of this lane's distance position at offset 0.
-    const int trow0 = wave * ROWS + S;  // + r + qy
-    const int tcol0 = lane + S;          // + qx
-    // Gather column of the output pixel: lane - P + S (+/- qx).  Lanes below 2P own no output and
-    // read a clamped column so every LDS read stays inside the tile.
-    const int gcol0 = max(lane, P) - P + S;
+    // Sample of this lane's first distance column, and of its first output pixel (the distance row P
+    // above, P columns on), at offset 0; lanes below 2P own no output and read rows inside the tile.
+    const int dist0 = (lane + S) * pitch + wave * COLS + S;
+    const int gather0 = (max(lane, P) - P + S) * pitch + wave * COLS + P + S;
     // This wave's share of the offsets: the rows qy of part `part` of SPLIT consecutive runs of
-    // offset rows (a test inside the loop for a finer split cost the loop its shape and doubled its
-    // registers).
+    // offset rows.
     const int qy_lo = -S + part * side / SPLIT, qy_hi = -S + (part + 1) * side / SPLIT;
     for (int qy = qy_lo; qy < qy_hi; ++qy) {
         for (int qx = -S; qx <= S; ++qx) {
             if (!PAIR && qx == 0 && qy == 0) continue;
             const float off = PAIR ? w.offset : lut[(qy + S) * side + (qx + S)];
-            float hf[DR], hb[DR];
+            const int q = qy * pitch + qx;
+            float wf[COLS];
+            offset_weights<C, P, COLS>(tf + (size_t)(dist0 + q) * C, cen, scale, off, h2l, wf);
+            const float *gf = tf + (size_t)(gather0 + q) * C;
+            if constexpr (PAIR) {
+                float wb[COLS];
+                offset_weights<C, P, COLS>(tb + (size_t)(dist0 - q) * C, cen, scale, off, h2l, wb);
+                const float *gb = tb + (size_t)(gather0 - q) * C;
 #pragma unroll
-            for (int r = 0; r < DR; ++r) {
-                const float *nf = tf + ((size_t)(trow0 + r + qy) * tcols + (tcol0 + qx)) * C;
-                float df = 0.0f;
-#pragma unroll
-                for (int c = 0; c < C; ++c) {
-                    const float e = cen[r][c] - nf[c];
-                    df += e * e;
-                }
-                df *= scale;
-                float a = df;
-#pragma unroll
-                for (int k = 0; k < 2 * P; ++k) a = df + wave_shr1(a);
-                hf[r] = a;
-                if (PAIR) {
-                    const float *nb = tb + ((size_t)(trow0 + r - qy) * tcols + (tcol0 - qx)) * C;
-                    float db = 0.0f;
-#pragma unroll
-                    for (int c = 0; c < C; ++c) {
-                        const float e = cen[r][c] - nb[c];
-                        db += e * e;
+                for (int j = 0; j < COLS; ++j) {
+                    float cf = wf[j], cb = wb[j], both;
+                    if constexpr (CONF) {
+                        cf = wf[j] * conf_fv[j];
+                        cb = wb[j] * conf_bv[j];
+                        both = fmaf(conf_fv[j], wf[j], cb);
+                    } else {
+                        both = cf + cb;
                     }
-                    db *= scale;
-                    float b = db;
 #pragma unroll
-                    for (int k = 0; k < 2 * P; ++k) b = db + wave_shr1(b);
-                    hb[r] = b;
+                    for (int c = 0; c < C; ++c)
+                        acc[j][c] = fmaf(gb[j * C + c], cb, fmaf(gf[j * C + c], cf, acc[j][c]));
+                    ws[j] += both;
+                    mw[j] = fmaxf(mw[j], fmaxf(cf, cb));
                 }
-            }
+            } else {
 #pragma unroll
-            for (int j = 0; j < ROWS; ++j) {
-                float Df = 0.0f;
+                for (int j = 0; j < COLS; ++j) {
 #pragma unroll
-                for (int k = 0; k <= 2 * P; ++k) Df += hf[j + k];
-                float wf = __builtin_amdgcn_exp2f(-fmaxf(Df - off, 0.0f) * h2l);
-                if (CONF) wf *= conf_fv[j];
-                // The gathered neighbour sits at the output pixel plus q: distance row j+P, column lane-P.
-                const float *gf = tf + ((size_t)(trow0 + j + P + qy) * tcols + (gcol0 + qx)) * C;
-                if (PAIR) {
-                    float Db = 0.0f;
-#pragma unroll
-                    for (int k = 0; k <= 2 * P; ++k) Db += hb[j + k];
-                    float wb = __builtin_amdgcn_exp2f(-fmaxf(Db - off, 0.0f) * h2l);
-                    if (CONF) wb *= conf_bv[j];
-                    const float *gb = tb + ((size_t)(trow0 + j + P - qy) * tcols + (gcol0 - qx)) * C;
-#pragma unroll
-                    for (int c = 0; c < C; ++c) acc[j][c] = acc[j][c] + gf[c] * wf + gb[c] * wb;
-                    ws[j] += wf + wb;
-                    mw[j] = fmaxf(mw[j], fmaxf(wf, wb));
-                } else {
-#pragma unroll
-                    for (int c = 0; c < C; ++c) acc[j][c] += gf[c] * wf;
-                    ws[j] += wf;
-                    mw[j] = fmaxf(mw[j], wf);
+                    for (int c = 0; c < C; ++c) acc[j][c] = fmaf(gf[j * C + c], wf[j], acc[j][c]);
+                    ws[j] += wf[j];
+                    mw[j] = fmaxf(mw[j], wf[j]);
                 }
             }
         }
     }
 }
 
-// Adds the window sums of parts 1 .. SPLIT-1 into part 0's, in part order, through `red`: LDS of
-// (SPLIT - 1) * WV * kCombineRows * (C + 2) * 64 floats, kCombineRows output rows at a time (the
-// tiles are done with, so the caller passes their memory).  Every wave of the workgroup calls it;
-// part 0 holds the totals afterwards.
-constexpr int kCombineRows = 4;
-
-template <int C, int ROWS, int WV, int SPLIT>
-__device__ __forceinline__ void combine_parts(float *red, int wave, int lane, int part, float (&acc)[ROWS][C],
-                                              float (&ws)[ROWS], float (&mw)[ROWS])
+// Hands the window sums from the lanes that walked them to the threads that finish them: each field
+// (the C channel sums, the weight sum, the largest weight) passes through `red`, LDS of SPLIT x 64 x
+// (kWidth + 1) floats (the tiles are done with, so the caller passes their memory), and element k of
+// a thread is pixel (t + k kThreads) of the 64 x kWidth grid, its parts joined in part order.  Every
+// thread of the workgroup calls it.
+template <int C, int P, int COLS, int WX, int SPLIT>
+__device__ __forceinline__ void join_parts(float *red, int wave, int lane, int part, const float (&acc)[COLS][C],
+                                           const float (&ws)[COLS], const float (&mw)[COLS],
+                                           float (&out)[Shape<C, P, COLS, WX, SPLIT>::kElems][C + 2])
 {
-    if constexpr (SPLIT > 1) {
-        constexpr int CR = ROWS < kCombineRows ? ROWS : kCombineRows, F = CR * (C + 2);
+    using T = Shape<C, P, COLS, WX, SPLIT>;
+    constexpr int kPitch = T::kWidth + 1, kPart = 64 * kPitch;
 #pragma unroll
-        for (int j0 = 0; j0 < ROWS; j0 += CR) {
-            __syncthreads();  // every wave is done with the tiles, or part 0 with the last rows
-            if (part > 0) {
-                float *dst = red + ((size_t)((part - 1) * WV + wave) * F) * 64 + lane;
+    for (int f = 0; f < C + 2; ++f) {
+        __syncthreads();  // every wave is done with the tiles, or with the last field
+        float *dst = red + part * kPart + lane * kPitch + wave * COLS;
 #pragma unroll
-                for (int j = 0; j < CR; ++j) {
+        for (int j = 0; j < COLS; ++j) dst[j] = f < C ? acc[j][f < C ? f : 0] : (f == C ? ws[j] : mw[j]);
+        __syncthreads();
 #pragma unroll
-                    for (int c = 0; c < C; ++c) dst[(size_t)(j * (C + 2) + c) * 64] = acc[j0 + j][c];
-                    dst[(size_t)(j * (C + 2) + C) * 64] = ws[j0 + j];
-                    dst[(size_t)(j * (C + 2) + C + 1) * 64] = mw[j0 + j];
-                }
-            }
-            __syncthreads();
-            if (part == 0) {
+        for (int k = 0; k < T::kElems; ++k) {
+            const int e = min((int)threadIdx.x + k * T::kThreads, 64 * T::kWidth - 1);
+            const float *src = red + (e / T::kWidth) * kPitch + e % T::kWidth;
+            float v = src[0];
 #pragma unroll
-                for (int p = 1; p < SPLIT; ++p) {
-                    const float *src = red + ((size_t)((p - 1) * WV + wave) * F) * 64 + lane;
-#pragma unroll
-                    for (int j = 0; j < CR; ++j) {
-#pragma unroll
-                        for (int c = 0; c < C; ++c)
-                            acc[j0 + j][c] = acc[j0 + j][c] + src[(size_t)(j * (C + 2) + c) * 64];
-                        ws[j0 + j] = ws[j0 + j] + src[(size_t)(j * (C + 2) + C) * 64];
-                        mw[j0 + j] = fmaxf(mw[j0 + j], src[(size_t)(j * (C + 2) + C + 1) * 64]);
-                    }
-                }
-            }
+            for (int p = 1; p < SPLIT; ++p) v = f <= C ? v + src[p * kPart] : fmaxf(v, src[p * kPart]);
+            out[k][f] = v;
         }
     }
 }
 
-// The centre values of this lane's distance column, one per distance row, and the confidence of
-// the blocks its output rows fall in.
-template <int C, int P, int ROWS>
-__device__ __forceinline__ void load_centre(const NlmWindow &w, const float *__restrict__ centre, int X0, int Y0,
-                                            int wave, int lane, float (&cen)[ROWS + 2 * P][C])
+// The pixel of element k of this thread, or false where it lies outside the tile's outputs.
+template <int P, typename T>
+__device__ __forceinline__ bool element_pixel(int k, int X0, int Y0, int W, int H, size_t &p)
 {
-    const int xd = X0 - P + lane;
-    const int ybase = Y0 + wave * ROWS - P;
-#pragma unroll
-    for (int r = 0; r < ROWS + 2 * P; ++r) {
-        const float *src = centre + ((size_t)clampi(ybase + r, w.H - 1) * w.W + clampi(xd, w.W - 1)) * C;
-#pragma unroll
-        for (int c = 0; c < C; ++c) cen[r][c] = src[c];
-    }
+    const int e = (int)threadIdx.x + k * T::kThreads, row = e / T::kWidth;
+    const int ox = X0 + e % T::kWidth, oy = Y0 - 2 * P + row;
+    p = (size_t)oy * W + ox;
+    return row >= 2 * P && row < 64 && ox < W && oy < H;
 }
 
-template <int ROWS>
-__device__ __forceinline__ void load_conf(const NlmWindow &w, const float *__restrict__ conf, int ox, int Y0, int wave,
-                                          float (&out)[ROWS])
+// The centre samples of this lane's distance row from the staged centre tile.
+template <int C, int P, int COLS>
+__device__ __forceinline__ void read_centre(const float *tile, int pitch, int S, int wave, int lane,
+                                            float (&cen)[COLS + 2 * P][C])
 {
-    const int bcol = min(clampi(ox, w.W - 1) / w.step, w.blocks_x - 1);
+    const float *src = tile + (size_t)((lane + S) * pitch + wave * COLS + S) * C;
 #pragma unroll
-    for (int j = 0; j < ROWS; ++j) {
-        const int oy = clampi(Y0 + wave * ROWS + j, w.H - 1);
-        out[j] = conf[min(oy / w.step, w.blocks_y - 1) * w.blocks_x + bcol];
-    }
+    for (int i = 0; i < COLS + 2 * P; ++i)
+#pragma unroll
+        for (int c = 0; c < C; ++c) cen[i][c] = src[i * C + c];
 }
 
-template <int C, int P, int WV, int ROWS, bool PAIR, bool CONF, int SPLIT>
-__global__ __launch_bounds__(WV * SPLIT * 64) void k_nlm(NlmWindow w, const float *__restrict__ centre,
+// The confidence of the blocks this lane's output pixels fall in.
+template <int COLS>
+__device__ __forceinline__ void load_conf(const NlmWindow &w, const float *__restrict__ conf, int ox, int oy,
+                                          float (&out)[COLS])
+{
+    const float *row = conf + (size_t)min(clampi(oy, w.H - 1) / w.step, w.blocks_y - 1) * w.blocks_x;
+#pragma unroll
+    for (int j = 0; j < COLS; ++j) out[j] = row[min(clampi(ox + j, w.W - 1) / w.step, w.blocks_x - 1)];
+}
+
+template <int C, int P, int COLS, int WX, bool PAIR, bool CONF, int SPLIT>
+__global__ __launch_bounds__(WX * SPLIT * 64) void k_nlm(NlmWindow w, const float *__restrict__ centre,
                                                              const float *__restrict__ fwd, const float *__restrict__ bwd,
                                                              const float *__restrict__ lut,
                                                              const float *__restrict__ conf_f,
                                                              const float *__restrict__ conf_b, float *__restrict__ accum,
                                                              float *__restrict__ wsum, float *__restrict__ maxw)
 {
+    using T = Shape<C, P, COLS, WX, SPLIT>;
     extern __shared__ float lds[];
     const int S = w.S, W = w.W, H = w.H;
-    // Wave (wave, part): row group `wave` of the workgroup's WV, offset part `part` of SPLIT.
-    const int lane = threadIdx.x & 63, wave = (threadIdx.x >> 6) % WV;
-    const int part = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6) / WV);  // uniform per wave
-    const int X0 = blockIdx.x * (64 - 2 * P);
-    const int Y0 = blockIdx.y * (WV * ROWS);
+    // Wave (wave, part): column run `wave` of the workgroup's WX, offset part `part` of SPLIT.
+    const int lane = threadIdx.x & 63, id = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int wave = id % WX, part = id / WX;
+    const int X0 = blockIdx.x * T::kWidth, Y0 = blockIdx.y * T::kRows;
 
-    // Neighbour tiles: columns X0-P-S .. X0-P+63+S, rows Y0-P-S .. Y0+WV*ROWS+P-1+S.
-    const int tcols = 64 + 2 * S, trows = WV * ROWS + 2 * P + 2 * S;
+    // Tiles: columns X0-P-S .. X0+kWidth+P-1+S, rows Y0-P-S .. Y0+63-P+S.
+    const int tcols = T::kWidth + 2 * P + 2 * S, trows = 64 + 2 * S, pitch = tile_pitch(T::kWidth, P, S);
     const int tx0 = X0 - P - S, ty0 = Y0 - P - S;
     float *tf = lds;
-    float *tb = lds + (size_t)tcols * trows * C;
-    stage_tile<C, WV * SPLIT>(tf, fwd, W, H, tx0, ty0, tcols, trows);
-    if (PAIR) stage_tile<C, WV * SPLIT>(tb, bwd, W, H, tx0, ty0, tcols, trows);
-    float cen[ROWS + 2 * P][C];
-    load_centre<C, P, ROWS>(w, centre, X0, Y0, wave, lane, cen);
+    float *tb = lds + (size_t)pitch * trows * C;
+    float cen[T::kDist][C];
+    stage_tile<C, T::kThreads, T::kStage>(tf, centre, W, H, tx0, ty0, tcols, trows, pitch);
     __syncthreads();
-
-    const int ox = X0 - 2 * P + lane;  // output column of this lane (valid for lane >= 2P)
-    float conf_fv[ROWS], conf_bv[ROWS];
-    if (CONF) {
-        load_conf<ROWS>(w, conf_f, ox, Y0, wave, conf_fv);
-        load_conf<ROWS>(w, conf_b, ox, Y0, wave, conf_bv);
+    read_centre<C, P, COLS>(tf, pitch, S, wave, lane, cen);
+    if (PAIR) {
+        __syncthreads();
+        stage_tile<C, T::kThreads, T::kStage>(tf, fwd, W, H, tx0, ty0, tcols, trows, pitch);
+        stage_tile<C, T::kThreads, T::kStage>(tb, bwd, W, H, tx0, ty0, tcols, trows, pitch);
+        __syncthreads();
     }
-    float acc[ROWS][C], ws[ROWS], mw[ROWS];
-    window_sums<C, P, ROWS, PAIR, CONF, SPLIT>(w, tf, tb, tcols, wave, lane, part, cen, lut, conf_fv, conf_bv, acc, ws,
+    float conf_fv[COLS], conf_bv[COLS];
+    if (CONF) {
+        load_conf<COLS>(w, conf_f, X0 + wave * COLS, Y0 - 2 * P + lane, conf_fv);
+        load_conf<COLS>(w, conf_b, X0 + wave * COLS, Y0 - 2 * P + lane, conf_bv);
+    }
+    float acc[COLS][C], ws[COLS], mw[COLS], out[T::kElems][C + 2];
+    window_sums<C, P, COLS, PAIR, CONF, SPLIT>(w, tf, tb, pitch, wave, lane, part, cen, lut, conf_fv, conf_bv, acc, ws,
                                                mw);
-    combine_parts<C, ROWS, WV, SPLIT>(lds, wave, lane, part, acc, ws, mw);
-
-    if (part != 0 || lane < 2 * P || ox >= W) return;
+    join_parts<C, P, COLS, WX, SPLIT>(lds, wave, lane, part, acc, ws, mw, out);
 #pragma unroll
-    for (int j = 0; j < ROWS; ++j) {
-        const int oy = Y0 + wave * ROWS + j;
-        if (oy >= H) break;
-        const size_t p = (size_t)oy * W + ox;
+    for (int k = 0; k < T::kElems; ++k) {
+        size_t p;
+        if (!element_pixel<P, T>(k, X0, Y0, W, H, p)) continue;
 #pragma unroll
-        for (int c = 0; c < C; ++c) accum[p * C + c] += acc[j][c];
-        wsum[p] += ws[j];
-        maxw[p] = fmaxf(maxw[p], mw[j]);
+        for (int c = 0; c < C; ++c) accum[p * C + c] += out[k][c];
+        wsum[p] += out[k][C];
+        maxw[p] = fmaxf(maxw[p], out[k][C + 1]);
     }
 }
 
@@ -280,81 +322,75 @@ __global__ __launch_bounds__(WV * SPLIT * 64) void k_nlm(NlmWindow w, const floa
 // form adds every launch's sums to accumulators that start at zero), so the output is bit-identical
 // to the plain launches' while the accumulators never reach memory.  The pair tiles are re-staged
 // per pair; the single window stages the centre frame into the first of them.
-template <int C, int P, int WV, int ROWS, bool CONF, int SPLIT>
-__global__ __launch_bounds__(WV * SPLIT * 64) void k_nlm_window(NlmWindow w, NlmFrames f,
+template <int C, int P, int COLS, int WX, bool CONF, int SPLIT>
+__global__ __launch_bounds__(WX * SPLIT * 64) void k_nlm_window(NlmWindow w, NlmFrames f,
                                                                 const float *__restrict__ centre,
                                                                 const float *__restrict__ lut, float self_weight,
                                                                 float *__restrict__ out)
 {
+    using T = Shape<C, P, COLS, WX, SPLIT>;
     extern __shared__ float lds[];
     const int S = w.S, W = w.W, H = w.H;
-    const int lane = threadIdx.x & 63, wave = (threadIdx.x >> 6) % WV;
-    const int part = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6) / WV);  // uniform per wave
-    const int X0 = blockIdx.x * (64 - 2 * P);
-    const int Y0 = blockIdx.y * (WV * ROWS);
-    const int tcols = 64 + 2 * S, trows = WV * ROWS + 2 * P + 2 * S;
+    const int lane = threadIdx.x & 63, id = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int wave = id % WX, part = id / WX;
+    const int X0 = blockIdx.x * T::kWidth, Y0 = blockIdx.y * T::kRows;
+    const int tcols = T::kWidth + 2 * P + 2 * S, trows = 64 + 2 * S, pitch = tile_pitch(T::kWidth, P, S);
     const int tx0 = X0 - P - S, ty0 = Y0 - P - S;
     float *tf = lds;
-    float *tb = lds + (size_t)tcols * trows * C;
-    float cen[ROWS + 2 * P][C];
-    load_centre<C, P, ROWS>(w, centre, X0, Y0, wave, lane, cen);
-    const int ox = X0 - 2 * P + lane;
+    float *tb = lds + (size_t)pitch * trows * C;
+    float cen[T::kDist][C];
+    stage_tile<C, T::kThreads, T::kStage>(tf, centre, W, H, tx0, ty0, tcols, trows, pitch);
+    __syncthreads();
+    read_centre<C, P, COLS>(tf, pitch, S, wave, lane, cen);
 
-    float tacc[ROWS][C], tws[ROWS], tmw[ROWS];
+    float total[T::kElems][C + 2];
 #pragma unroll
-    for (int j = 0; j < ROWS; ++j) {
+    for (int k = 0; k < T::kElems; ++k)
 #pragma unroll
-        for (int c = 0; c < C; ++c) tacc[j][c] = 0.0f;
-        tws[j] = 0.0f;
-        tmw[j] = 0.0f;
-    }
-    float acc[ROWS][C], ws[ROWS], mw[ROWS];
-    float conf_fv[ROWS], conf_bv[ROWS];
+        for (int c = 0; c < C + 2; ++c) total[k][c] = 0.0f;
+    float acc[COLS][C], ws[COLS], mw[COLS], sums[T::kElems][C + 2];
+    float conf_fv[COLS], conf_bv[COLS];
+    auto join = [&] {
+        join_parts<C, P, COLS, WX, SPLIT>(lds, wave, lane, part, acc, ws, mw, sums);
+#pragma unroll
+        for (int k = 0; k < T::kElems; ++k) {
+#pragma unroll
+            for (int c = 0; c <= C; ++c) total[k][c] = total[k][c] + sums[k][c];
+            total[k][C + 1] = fmaxf(total[k][C + 1], sums[k][C + 1]);
+        }
+    };
     for (int k = 0; k < f.pairs; ++k) {
-        if (k > 0) __syncthreads();  // every wave is done with the previous pair's tiles
-        stage_tile<C, WV * SPLIT>(tf, f.fwd[k], W, H, tx0, ty0, tcols, trows);
-        stage_tile<C, WV * SPLIT>(tb, f.bwd[k], W, H, tx0, ty0, tcols, trows);
+        __syncthreads();  // every wave is done with the centre tile, or the previous pair's sums
+        stage_tile<C, T::kThreads, T::kStage>(tf, f.fwd[k], W, H, tx0, ty0, tcols, trows, pitch);
+        stage_tile<C, T::kThreads, T::kStage>(tb, f.bwd[k], W, H, tx0, ty0, tcols, trows, pitch);
         __syncthreads();
         if (CONF) {
-            load_conf<ROWS>(w, f.conf_f[k], ox, Y0, wave, conf_fv);
-            load_conf<ROWS>(w, f.conf_b[k], ox, Y0, wave, conf_bv);
+            load_conf<COLS>(w, f.conf_f[k], X0 + wave * COLS, Y0 - 2 * P + lane, conf_fv);
+            load_conf<COLS>(w, f.conf_b[k], X0 + wave * COLS, Y0 - 2 * P + lane, conf_bv);
         }
-        window_sums<C, P, ROWS, true, CONF, SPLIT>(w, tf, tb, tcols, wave, lane, part, cen, nullptr, conf_fv, conf_bv,
+        window_sums<C, P, COLS, true, CONF, SPLIT>(w, tf, tb, pitch, wave, lane, part, cen, nullptr, conf_fv, conf_bv,
                                                    acc, ws, mw);
-        combine_parts<C, ROWS, WV, SPLIT>(lds, wave, lane, part, acc, ws, mw);
-#pragma unroll
-        for (int j = 0; j < ROWS; ++j) {
-#pragma unroll
-            for (int c = 0; c < C; ++c) tacc[j][c] = tacc[j][c] + acc[j][c];
-            tws[j] = tws[j] + ws[j];
-            tmw[j] = fmaxf(tmw[j], mw[j]);
-        }
+        join();
     }
-    if (f.pairs > 0) __syncthreads();
-    stage_tile<C, WV * SPLIT>(tf, centre, W, H, tx0, ty0, tcols, trows);
-    __syncthreads();
-    window_sums<C, P, ROWS, false, false, SPLIT>(w, tf, tf, tcols, wave, lane, part, cen, lut, conf_fv, conf_bv, acc,
+    if (f.pairs > 0) {
+        __syncthreads();
+        stage_tile<C, T::kThreads, T::kStage>(tf, centre, W, H, tx0, ty0, tcols, trows, pitch);
+        __syncthreads();
+    }
+    window_sums<C, P, COLS, false, false, SPLIT>(w, tf, tf, pitch, wave, lane, part, cen, lut, conf_fv, conf_bv, acc,
                                                  ws, mw);
-    combine_parts<C, ROWS, WV, SPLIT>(lds, wave, lane, part, acc, ws, mw);
-
-    if (part != 0 || lane < 2 * P || ox >= W) return;
+    join();
     // The finish (accumulate.rs:54-101), as k_finish computes it.
 #pragma unroll
-    for (int j = 0; j < ROWS; ++j) {
-        const int oy = Y0 + wave * ROWS + j;
-        if (oy >= H) break;
-        float a[C];
-#pragma unroll
-        for (int c = 0; c < C; ++c) a[c] = tacc[j][c] + acc[j][c];
-        const float wsum = tws[j] + ws[j];
-        const float maxw = fmaxf(tmw[j], mw[j]);
-        const size_t p = (size_t)oy * W + ox;
-        const float sw = self_weight * maxw;
-        const float den = sw + wsum;
+    for (int k = 0; k < T::kElems; ++k) {
+        size_t p;
+        if (!element_pixel<P, T>(k, X0, Y0, W, H, p)) continue;
+        const float sw = self_weight * total[k][C + 1];
+        const float den = sw + total[k][C];
         if (den > 1e-30f) {
             const float inv = 1.0f / den;
 #pragma unroll
-            for (int c = 0; c < C; ++c) out[p * C + c] = (centre[p * C + c] * sw + a[c]) * inv;
+            for (int c = 0; c < C; ++c) out[p * C + c] = (centre[p * C + c] * sw + total[k][c]) * inv;
         } else {
 #pragma unroll
             for (int c = 0; c < C; ++c) out[p * C + c] = centre[p * C + c];
@@ -381,35 +417,32 @@ __global__ __launch_bounds__(256) void k_finish(const float *__restrict__ frame,
     }
 }
 
-// Row groups per workgroup: pairs of two-channel frames stage two tiles of twice the width, so they
-// take half the rows to keep the LDS footprint near that of a luma pass; and a workgroup holds at
-// most eight waves (row groups x offset parts), four for two channels, whose windows with large
-// patches need more than 256 VGPRs.
+// Waves side by side in a workgroup: four, within eight waves (column runs x offset parts); pairs of
+// two-channel frames stage two tiles of twice the width, so they take two, within four waves.
 constexpr int waves_for(int C, bool pair, int split)
 {
     const int base = (pair && C == 2) ? 2 : 4, cap = C == 2 ? 4 : 8;
-    return base * split > cap ? (cap / split > 0 ? cap / split : 1) : base;
+    return base * split > cap ? cap / split : base;
 }
 
-// Offset parts per row group: each workgroup runs SPLIT waves per row group, each on a consecutive
+// Offset parts: each workgroup runs SPLIT waves per column run, each on a consecutive
 // run of the window's offset rows, so a frame puts SPLIT times the waves on the chip.  Planes up to
-// 2^20 pixels, which would leave SIMDs idle otherwise, take four (one channel) or two (two
-// channels, whose workgroups hold at most four waves); larger ones fill the chip with one (on an
-// MI355X: 640x360 spatial luma 12.3k frames/s against 6.3k at one part; 1920x1080 4:2:0 at
-// temporal radius 2, 643 frames/s against 596 at one part everywhere, 610 with four for chroma and
-// ≈620 with two for luma).  The part sums add in part order, the same for every tile shape and both
-// launch forms, which therefore stay bit-identical.
-inline int offset_split(int W, int H, int C) { return (size_t)W * H <= (1u << 20) ? (C == 1 ? 4 : 2) : 1; }
+// 2^20 pixels take four (one channel) or two (two channels, whose workgroups hold at most four waves);
+// larger ones have waves enough with one: 640x360 makes 480 waves of eight columns at one part, 1920x1080
+// about 4500 (when the line was drawn 640x360 ran 12.3k frames/s against 6.3k at one part, 1920x1080
+// 4:2:0 643 frames/s against 620 with two parts for luma).  The part sums add in part order, the same
+// for every tile shape and both launch forms, which therefore stay bit-identical: a plane's split is
+// part of its result.
+constexpr int offset_parts(int C) { return C == 1 ? 4 : 2; }
+inline int offset_split(int W, int H, int C) { return (size_t)W * H <= (1u << 20) ? offset_parts(C) : 1; }
 
-// LDS of a workgroup: its tile(s), or the part sums while they combine, whichever is larger.
-size_t tile_bytes(int C, int P, int S, bool pair, int rows, int split)
+// LDS of a workgroup: its tile(s), or the part sums of one field while they join, whichever is larger.
+size_t tile_bytes(int C, int P, int S, bool pair, int cols, int split, int waves)
 {
-    const int wv = waves_for(C, pair, split);
-    const size_t one = (size_t)(64 + 2 * S) * (wv * rows + 2 * P + 2 * S) * C * sizeof(float);
-    const size_t tiles = pair ? 2 * one : one;
-    const int cr = rows < kCombineRows ? rows : kCombineRows;
-    const size_t parts = (size_t)(split - 1) * wv * cr * (C + 2) * 64 * sizeof(float);
-    return tiles > parts ? tiles : parts;
+    const int width = waves * cols;
+    const size_t one = (size_t)tile_pitch(width, P, S) * (64 + 2 * S) * C * sizeof(float);
+    const size_t parts = (size_t)split * 64 * (width + 1) * sizeof(float);
+    return std::max(pair ? 2 * one : one, parts);
 }
 
 int device_lds_limit()
@@ -425,39 +458,36 @@ int device_lds_limit()
     return limit;
 }
 
-template <int C, int P, int ROWS, int SPLIT>
+template <int C, int P, int COLS, int SPLIT>
 hipError_t dispatch_split(const NlmWindow &w, const float *centre, const float *fwd, const float *bwd,
                           const float *lut, const float *cf, const float *cb, float *accum, float *wsum, float *maxw,
                           bool pair, bool conf, hipStream_t s)
 {
     constexpr int WS = waves_for(C, false, SPLIT), WP = waves_for(C, true, SPLIT);
-    const size_t lds = tile_bytes(C, P, w.S, pair, ROWS, SPLIT);
-    if (!pair) {
-        const dim3 grid(div_up(w.W, 64 - 2 * P), div_up(w.H, WS * ROWS));
-        k_nlm<C, P, WS, ROWS, false, false, SPLIT><<<grid, WS * SPLIT * 64, lds, s>>>(w, centre, fwd, bwd, lut, cf,
+    const size_t lds = tile_bytes(C, P, w.S, pair, COLS, SPLIT, pair ? WP : WS);
+    const dim3 grid(div_up(w.W, (pair ? WP : WS) * COLS), div_up(w.H, 64 - 2 * P));
+    if (!pair)
+        k_nlm<C, P, COLS, WS, false, false, SPLIT><<<grid, WS * SPLIT * 64, lds, s>>>(w, centre, fwd, bwd, lut, cf,
                                                                                      cb, accum, wsum, maxw);
-    } else {
-        const dim3 grid(div_up(w.W, 64 - 2 * P), div_up(w.H, WP * ROWS));
-        if (conf)
-            k_nlm<C, P, WP, ROWS, true, true, SPLIT><<<grid, WP * SPLIT * 64, lds, s>>>(w, centre, fwd, bwd, lut, cf,
-                                                                                       cb, accum, wsum, maxw);
-        else
-            k_nlm<C, P, WP, ROWS, true, false, SPLIT><<<grid, WP * SPLIT * 64, lds, s>>>(w, centre, fwd, bwd, lut, cf,
-                                                                                        cb, accum, wsum, maxw);
-    }
+    else if (conf)
+        k_nlm<C, P, COLS, WP, true, true, SPLIT><<<grid, WP * SPLIT * 64, lds, s>>>(w, centre, fwd, bwd, lut, cf,
+                                                                                   cb, accum, wsum, maxw);
+    else
+        k_nlm<C, P, COLS, WP, true, false, SPLIT><<<grid, WP * SPLIT * 64, lds, s>>>(w, centre, fwd, bwd, lut, cf,
+                                                                                    cb, accum, wsum, maxw);
     return hipGetLastError();
 }
 
-template <int C, int P, int ROWS>
-hipError_t dispatch_rows(const NlmWindow &w, const float *centre, const float *fwd, const float *bwd, const float *lut,
+// One channel splits its offsets over four parts or none, two channels over two or none.
+template <int C, int P, int COLS>
+hipError_t dispatch_cols(const NlmWindow &w, const float *centre, const float *fwd, const float *bwd, const float *lut,
                          const float *cf, const float *cb, float *accum, float *wsum, float *maxw, bool pair, bool conf,
                          hipStream_t s)
 {
-    switch (offset_split(w.W, w.H, C)) {
-    case 4: return dispatch_split<C, P, ROWS, 4>(w, centre, fwd, bwd, lut, cf, cb, accum, wsum, maxw, pair, conf, s);
-    case 2: return dispatch_split<C, P, ROWS, 2>(w, centre, fwd, bwd, lut, cf, cb, accum, wsum, maxw, pair, conf, s);
-    default: return dispatch_split<C, P, ROWS, 1>(w, centre, fwd, bwd, lut, cf, cb, accum, wsum, maxw, pair, conf, s);
-    }
+    if (offset_split(w.W, w.H, C) > 1)
+        return dispatch_split<C, P, COLS, offset_parts(C)>(w, centre, fwd, bwd, lut, cf, cb, accum, wsum, maxw, pair,
+                                                           conf, s);
+    return dispatch_split<C, P, COLS, 1>(w, centre, fwd, bwd, lut, cf, cb, accum, wsum, maxw, pair, conf, s);
 }
 
 template <int C, int P>
@@ -466,9 +496,9 @@ hipError_t dispatch(const NlmWindow &w, const float *centre, const float *fwd, c
                     int variant, hipStream_t s)
 {
     switch (variant) {
-    case 1: return dispatch_rows<C, P, 8>(w, centre, fwd, bwd, lut, cf, cb, accum, wsum, maxw, pair, conf, s);
-    case 2: return dispatch_rows<C, P, 4>(w, centre, fwd, bwd, lut, cf, cb, accum, wsum, maxw, pair, conf, s);
-    default: return dispatch_rows<C, P, 16>(w, centre, fwd, bwd, lut, cf, cb, accum, wsum, maxw, pair, conf, s);
+    case 1: return dispatch_cols<C, P, 4>(w, centre, fwd, bwd, lut, cf, cb, accum, wsum, maxw, pair, conf, s);
+    case 2: return dispatch_cols<C, P, 2>(w, centre, fwd, bwd, lut, cf, cb, accum, wsum, maxw, pair, conf, s);
+    default: return dispatch_cols<C, P, 8>(w, centre, fwd, bwd, lut, cf, cb, accum, wsum, maxw, pair, conf, s);
     }
 }
 
@@ -491,32 +521,30 @@ hipError_t dispatch_p(const NlmWindow &w, const float *centre, const float *fwd,
     }
 }
 
-template <int C, int P, int ROWS, int SPLIT>
+template <int C, int P, int COLS, int SPLIT>
 hipError_t dispatch_window_split(const NlmWindow &w, const NlmFrames &f, const float *centre, const float *lut,
                                  float self_weight, float *out, hipStream_t s)
 {
-    constexpr int WV = waves_for(C, true, SPLIT);
-    const size_t lds = tile_bytes(C, P, w.S, true, ROWS, SPLIT);
-    const dim3 grid(div_up(w.W, 64 - 2 * P), div_up(w.H, WV * ROWS));
+    constexpr int WX = waves_for(C, true, SPLIT);
+    const size_t lds = tile_bytes(C, P, w.S, f.pairs > 0, COLS, SPLIT, WX);
+    const dim3 grid(div_up(w.W, WX * COLS), div_up(w.H, 64 - 2 * P));
     const bool conf = f.pairs > 0 && f.conf_f[0] != nullptr;
     if (conf)
-        k_nlm_window<C, P, WV, ROWS, true, SPLIT><<<grid, WV * SPLIT * 64, lds, s>>>(w, f, centre, lut, self_weight,
+        k_nlm_window<C, P, COLS, WX, true, SPLIT><<<grid, WX * SPLIT * 64, lds, s>>>(w, f, centre, lut, self_weight,
                                                                                     out);
     else
-        k_nlm_window<C, P, WV, ROWS, false, SPLIT><<<grid, WV * SPLIT * 64, lds, s>>>(w, f, centre, lut, self_weight,
+        k_nlm_window<C, P, COLS, WX, false, SPLIT><<<grid, WX * SPLIT * 64, lds, s>>>(w, f, centre, lut, self_weight,
                                                                                      out);
     return hipGetLastError();
 }
 
-template <int C, int P, int ROWS>
+template <int C, int P, int COLS>
 hipError_t dispatch_window(const NlmWindow &w, const NlmFrames &f, const float *centre, const float *lut,
                            float self_weight, float *out, hipStream_t s)
 {
-    switch (offset_split(w.W, w.H, C)) {
-    case 4: return dispatch_window_split<C, P, ROWS, 4>(w, f, centre, lut, self_weight, out, s);
-    case 2: return dispatch_window_split<C, P, ROWS, 2>(w, f, centre, lut, self_weight, out, s);
-    default: return dispatch_window_split<C, P, ROWS, 1>(w, f, centre, lut, self_weight, out, s);
-    }
+    if (offset_split(w.W, w.H, C) > 1)
+        return dispatch_window_split<C, P, COLS, offset_parts(C)>(w, f, centre, lut, self_weight, out, s);
+    return dispatch_window_split<C, P, COLS, 1>(w, f, centre, lut, self_weight, out, s);
 }
 
 template <int C>
@@ -547,12 +575,8 @@ hipError_t dispatch_window_p(const NlmWindow &w, const NlmFrames &f, const float
 bool nlm_supported(int C, int P, int S)
 {
     return (C == 1 || C == 2) && P >= 0 && P <= kMaxP && S >= 0 && S <= kMaxS &&
-           tile_bytes(C, P, S, true, 16, 2) <= (size_t)device_lds_limit() &&
-           tile_bytes(C, P, S, false, 16, 2) <= (size_t)device_lds_limit() &&
-           tile_bytes(C, P, S, true, 16, 4) <= (size_t)device_lds_limit() &&
-           tile_bytes(C, P, S, false, 16, 4) <= (size_t)device_lds_limit();
+           tile_bytes(C, P, S, true, 8, 1, waves_for(C, true, 1)) <= (size_t)device_lds_limit();
 }
-int nlm_variant_rows(int variant) { return variant == 1 ? 8 : (variant == 2 ? 4 : 16); }
 
 hipError_t launch_nlm_single(const NlmWindow &w, const float *frame, const float *lut, float *accum, float *wsum,
                              float *maxw, hipStream_t s, int variant)
