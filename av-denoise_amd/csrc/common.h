@@ -31,11 +31,14 @@ struct NlmWindow {
 // `variant` picks the columns each lane walks (0: 8, 1: 4, 2: 2); every variant gives bit-identical
 // sums, so the tuner may choose any (kNlmVariants of them).
 constexpr int kNlmVariants = 3;
+// A `fresh` window starts the accumulators instead of adding to them; a single window with `out`
+// finishes the frame there (as launch_nlm_finish would) instead of storing its sums.
 hipError_t launch_nlm_single(const NlmWindow &w, const float *frame, const float *lut, float *accum, float *wsum,
-                             float *maxw, hipStream_t s, int variant = 0);
+                             float *maxw, hipStream_t s, int variant = 0, bool fresh = false, float self_weight = 0.0f,
+                             float *out = nullptr);
 hipError_t launch_nlm_pair(const NlmWindow &w, const float *centre, const float *fwd, const float *bwd,
                            const float *conf_f, const float *conf_b, float *accum, float *wsum, float *maxw,
-                           hipStream_t s, int variant = 0);
+                           hipStream_t s, int variant = 0, bool fresh = false);
 hipError_t launch_nlm_finish(const float *frame, const float *accum, const float *wsum, const float *maxw,
                              float self_weight, uint32_t pixels, int C, float *out, hipStream_t s);
 bool nlm_supported(int C, int P, int S);

@@ -657,7 +657,7 @@ uint32_t NlmPass::push(const avd_device_plane *planes)
 
 void NlmPass::push_context(const avd_device_plane *planes) { ingest(planes); }
 
-// run_windowed_kernels (nlmeans/dispatch/mod.rs:665-679): zero, pairs q_k = -r..-1, single, finish.
+// run_windowed_kernels (nlmeans/dispatch/mod.rs:665-679): pairs q_k = -r..-1, then single and finish.
 void NlmPass::denoise()
 {
     const size_t px = (size_t)W_ * H_;
@@ -716,22 +716,16 @@ void NlmPass::denoise()
         next_output_ = (next_output_ + 1) % 2;
         return;
     }
-    check_hip(launch_fill_u32(accum_.ptr, 0, px * C, stream_), "zero");
-    check_hip(launch_fill_u32(wsum_.ptr, 0, px, stream_), "zero");
-    check_hip(launch_fill_u32(maxw_.ptr, 0, px, stream_), "zero");
+    // The first window starts the accumulators and the single window, the last, finishes the frame.
     for (int qk = -(int)r_; qk < 0; ++qk)
         timed(AVD_STAGE_NLM_PAIR, px * window * 2 * nlm_candidate_ops(C, P_), stream_, "nlm pair", [&] {
             return launch_nlm_pair(w, cf, nb[qk + r_], nb[-qk + r_], conf_of(qk), conf_of(-qk), accum_.as<float>(),
-                                   wsum_.as<float>(), maxw_.as<float>(), stream_, variant_pair_);
+                                   wsum_.as<float>(), maxw_.as<float>(), stream_, variant_pair_, qk == -(int)r_);
         });
+    float *out = outputs_[next_output_].as<float>();
     timed(AVD_STAGE_NLM_SINGLE, px * (window - 1) * nlm_candidate_ops(C, P_), stream_, "nlm single", [&] {
         return launch_nlm_single(w, cf, lut_.as<float>(), accum_.as<float>(), wsum_.as<float>(), maxw_.as<float>(),
-                                 stream_, variant_single_);
-    });
-    float *out = outputs_[next_output_].as<float>();
-    timed(AVD_STAGE_NLM_FINISH, px, stream_, "nlm finish", [&] {
-        return launch_nlm_finish(cf, accum_.as<float>(), wsum_.as<float>(), maxw_.as<float>(), self_weight_,
-                                 (uint32_t)px, C, out, stream_);
+                                 stream_, variant_single_, r_ == 0, self_weight_, out);
     });
     ready_output_ = next_output_;
     next_output_ = (next_output_ + 1) % 2;

@@ -263,7 +263,8 @@ avd_status avd_engine_timing(avd_engine *engine, avd_timing *out);
 
 /* No counterpart in the reference, whose NLMeans launches once per temporal pair, once for the
  * single window and once for the finish (nlmeans/dispatch/mod.rs:665-679): an NLMeans engine
- * runs each frame's windows that way (AVD_NLM_FORM_PLAIN) or batched (AVD_NLM_FORM_BATCHED:
+ * runs each frame's windows that way, the finish with the single window
+ * (AVD_NLM_FORM_PLAIN), or batched (AVD_NLM_FORM_BATCHED:
  * every pair, the single window and the finish of a plane group in one launch, the window sums
  * kept on chip).  The outputs are bit-identical.  AVD_NLM_FORM_DEFAULT, the form an engine starts
  * in, batches spatial passes and keeps temporal ones plain (the faster of the two on an MI355X at
