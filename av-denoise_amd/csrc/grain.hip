@@ -271,13 +271,16 @@ __global__ __launch_bounds__(kReduceThreads) void k_grain_reduce(const float *__
 }
 
 // The AR(3) fit in f64 (undo_mean_removal, yule_walker, solve and quantise_ar, nl4d/grain/fit.rs:
-// 79-300): one wave per 47-value record.  Each of the 20 mean-removal rounds has lane l < 46
-// compute lag l's cell-mean term over the 15 x 15 cell offsets in the reference's order and lane 46
-// the zero lag's; elimination gives row r to lane r (the factors
-// first, then each row's update), the pivot is the last of equal maxima (as Iterator::max_by
-// keeps), back substitution and quantisation run in lane 0.  Every f64 operation is the
-// reference's, in its order, so the results are bit-identical.
-__device__ inline int fit_lane(int dy, int dx)
+// 79-300): one wave per 47-value record, its state in registers.  Each of the 20 mean-removal rounds
+// has lane l < 46 add lag l's cell-mean term over the 91 cell offsets that reach a measured lag, in the
+// reference's order: the lane's weights are 91 registers (zero where the offset lies past the cell) and
+// the lags broadcast reads.  In the solve lane r holds row r of the 24 x 25 system; a row swap only
+// exchanges the lanes' row numbers, the pivot is the last of equal maxima in row order (as
+// Iterator::max_by keeps), and its row reaches the others by v_readlane.  Every f64 operation is the
+// reference's, in its order, so the results are bit-identical.  Bound by the chain of 20 x 91 dependent
+// adds, which a record cannot shorten; a segment's records run side by side.  16 records: 351 us
+// with the index arithmetic, the system in LDS and the pivot in one lane, 32 us now.
+__device__ __forceinline__ constexpr int fit_lane(int dy, int dx)
 {
     if (dy < 0 || (dy == 0 && dx < 0)) {
         dy = -dy;
@@ -287,126 +290,145 @@ __device__ inline int fit_lane(int dy, int dx)
     return dy == 0 ? dx : 7 + (dy - 1) * 13 + dx + 6;
 }
 
-__device__ inline double cell_term(const double *rho, int dy, int dx)
+__device__ __forceinline__ double readlane_f64(double v, int lane)
 {
-    double total = 0.0;
-    for (int oy = -7; oy <= 7; ++oy)
-        for (int ox = -7; ox <= 7; ++ox) {
-            const int lane = fit_lane(dy + oy, dx + ox);
-            if (lane < 0) continue;
-            const double pairs = (double)((8 - abs(oy)) * (8 - abs(ox)));
-            total += pairs / 4096.0 * rho[lane];
-        }
-    return total;
+    const uint64_t u = __builtin_bit_cast(uint64_t, v);
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)u, lane);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(u >> 32), lane);
+    return __builtin_bit_cast(double, (uint64_t)hi << 32 | lo);
 }
+
+// AR_OFFSETS: dy -3..0, dx -3..3, the causal half.
+__device__ __forceinline__ constexpr int ar_dy(int i) { return i < 21 ? -3 + i / 7 : 0; }
+__device__ __forceinline__ constexpr int ar_dx(int i) { return i < 21 ? i % 7 - 3 : i - 24; }
+
+constexpr int kWeights = 24, kCellTerms = 7 * 13;
 
 __global__ __launch_bounds__(64) void k_grain_fit(const double *__restrict__ records, double *__restrict__ corrected,
                                                   double *__restrict__ weights, int32_t *__restrict__ quantised,
                                                   uint32_t *__restrict__ shifts, int32_t *__restrict__ solved)
 {
-    __shared__ double s_rho[kLags], s_next[kLags], s_m[24][25], s_factor[24], s_sol[24];
-    __shared__ int s_oy[24], s_ox[24], s_ok;
-    __shared__ double s_zero_term;
+    __shared__ __align__(16) double s_lag[kRecordLen + 1];
     const int lane = (int)threadIdx.x;
     const size_t r = blockIdx.x;
     const double *rec = records + r * kRecordLen;
-    double *cor = corrected + r * kRecordLen;
+    // One wave: LDS written by its lanes is read by them after a fence.
     auto sync = [] {
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
     };
-    if (lane < 24) {  // AR_OFFSETS: dy -3..0, dx -3..3, the causal half
-        const int k = lane < 21 ? lane : lane - 21, dy = lane < 21 ? -3 + k / 7 : 0;
-        s_oy[lane] = dy;
-        s_ox[lane] = lane < 21 ? k % 7 - 3 : -3 + k;
-    }
-    const double zero_lag = rec[0];
-    const double measured = lane < kLags ? rec[lane] / zero_lag : 0.0;
-    if (lane < kLags) s_rho[lane] = lane == 0 ? 1.0 : measured;
-    sync();
+    const double raw = lane < kRecordLen ? rec[lane] : 0.0;
+    const double zero_lag = readlane_f64(raw, 0);
+    double lag = raw;
     if (zero_lag > 0.0) {
         const int dy = lane < 7 ? 0 : lane < 20 ? 1 : lane < 33 ? 2 : 3;
         const int dx = lane < 7 ? lane : (lane - 7) % 13 - 6;
+        double share[kCellTerms];  // pairs / 4096 of cell offset (ty - dy, tx - dx)
+#pragma unroll
+        for (int k = 0; k < kCellTerms; ++k) {
+            const int oy = abs(k / 13 - 3 - dy), ox = abs(k % 13 - 6 - dx);
+            share[k] = oy <= 7 && ox <= 7 ? (double)((8 - oy) * (8 - ox)) / 4096.0 : 0.0;
+        }
+        const double measured = raw / zero_lag;
+        double rho = lane == 0 ? 1.0 : measured;
         for (int round = 0; round < 20; ++round) {
-            // Lane 46 computes the zero lag's term once for every lane.
-            const double term = lane < kLags ? cell_term(s_rho, dy, dx) : lane == kLags ? cell_term(s_rho, 0, 0) : 0.0;
-            if (lane == kLags) s_zero_term = term;
+            if (lane < kLags) s_lag[lane] = rho;
             sync();
-            if (lane < kLags) s_next[lane] = measured * (1.0 - s_zero_term) + term;
-            sync();
-            if (lane < kLags) s_rho[lane] = s_next[lane];
+            double term = 0.0;
+#pragma unroll
+            for (int k = 0; k < kCellTerms; ++k) term += share[k] * s_lag[fit_lane(k / 13 - 3, k % 13 - 6)];
+            rho = measured * (1.0 - readlane_f64(term, 0)) + term;  // lane 0's term is the zero lag's
             sync();
         }
-        if (lane < kLags) cor[lane] = s_rho[lane] * zero_lag;
-        if (lane == kLags) cor[kLags] = rec[kLags];
-    } else if (lane < kRecordLen) {
-        cor[lane] = rec[lane];
+        if (lane < kLags) lag = rho * zero_lag;
     }
-    // The corrected record, read back as the solve's input.
-    __shared__ double s_cor[kRecordLen];
-    if (lane < kLags) s_cor[lane] = zero_lag > 0.0 ? s_rho[lane] * zero_lag : rec[lane];
-    if (lane == kLags) s_cor[kLags] = rec[kLags];
-    sync();
-    const double pixels = s_cor[kLags];
-    if (lane == 0) s_ok = pixels > 0.0;
-    if (lane < 24 && pixels > 0.0) {
-        for (int j = 0; j < 24; ++j) s_m[lane][j] = s_cor[fit_lane(s_oy[lane] - s_oy[j], s_ox[lane] - s_ox[j])] / pixels;
-        s_m[lane][24] = s_cor[fit_lane(s_oy[lane], s_ox[lane])] / pixels;
+    if (lane < kRecordLen) {
+        corrected[r * kRecordLen + lane] = lag;
+        s_lag[lane] = lag;
     }
     sync();
-    for (int col = 0; col < 24 && s_ok; ++col) {
-        if (lane == 0) {
-            int pivot = col;
-            for (int i = col + 1; i < 24; ++i)
-                if (fabs(s_m[i][col]) >= fabs(s_m[pivot][col])) pivot = i;
-            if (fabs(s_m[pivot][col]) < 1e-18) s_ok = 0;
-            else if (pivot != col)
-                for (int j = 0; j < 25; ++j) {
-                    const double t = s_m[col][j];
-                    s_m[col][j] = s_m[pivot][j];
-                    s_m[pivot][j] = t;
+
+    const double pixels = s_lag[kLags];
+    bool ok = pixels > 0.0;
+    double mine = 0.0;  // lane i's weight
+    if (ok) {
+        const int row_id = lane < kWeights ? lane : 0;
+        const int row_dy = ar_dy(row_id), row_dx = ar_dx(row_id);
+        double m[kWeights + 1];
+#pragma unroll
+        for (int j = 0; j < kWeights; ++j) m[j] = s_lag[fit_lane(row_dy - ar_dy(j), row_dx - ar_dx(j))] / pixels;
+        m[kWeights] = s_lag[fit_lane(row_dy, row_dx)] / pixels;
+        int at = lane < kWeights ? lane : -1;  // the row number this lane's row has now
+        int order[kWeights];                   // the lane that holds row number i
+#pragma unroll
+        for (int col = 0; col < kWeights; ++col) {
+            if (!ok) break;
+            // The pivot: the last row of the largest magnitude, or row `col` itself when that is NaN.
+            const double a = fabs(m[col]);
+            const int here = __builtin_ctzll(__ballot(at == col));
+            double top = at >= col && !isnan(a) ? a : -1.0;
+#pragma unroll
+            for (int x = 1; x < 32; x <<= 1) top = fmax(top, __shfl_xor(top, x));
+            const double first = readlane_f64(a, here);
+            int pivot = here;
+            if (!isnan(first)) {
+                const double largest = readlane_f64(top, 0);
+                uint64_t tied = __ballot(at >= col && a == largest);
+                int row = -1;
+                while (tied) {  // ties are rare; the lanes' rows are in no order
+                    const int l = __builtin_ctzll(tied);
+                    const int l_row = __builtin_amdgcn_readlane(at, l);
+                    if (l_row > row) {
+                        row = l_row;
+                        pivot = l;
+                    }
+                    tied &= tied - 1;
                 }
+            }
+            pivot = __builtin_amdgcn_readfirstlane(pivot);
+            if (readlane_f64(a, pivot) < 1e-18) {
+                ok = false;
+                break;
+            }
+            const int pivot_row = __builtin_amdgcn_readlane(at, pivot);
+            if (lane == here) at = pivot_row;
+            if (lane == pivot) at = col;
+            order[col] = pivot;
+            const double head = readlane_f64(m[col], pivot);
+            if (at > col) {
+                const double factor = m[col] / head;
+#pragma unroll
+                for (int j = col; j <= kWeights; ++j) m[j] -= factor * readlane_f64(m[j], pivot);
+            }
         }
-        sync();
-        if (!s_ok) break;
-        if (lane > col && lane < 24) s_factor[lane] = s_m[lane][col] / s_m[col][col];
-        sync();
-        if (lane > col && lane < 24)
-            for (int j = col; j < 25; ++j) s_m[lane][j] -= s_factor[lane] * s_m[col][j];
-        sync();
+        if (ok) {
+            double sol[kWeights];
+#pragma unroll
+            for (int i = kWeights - 1; i >= 0; --i) {
+                double v = m[kWeights];
+#pragma unroll
+                for (int j = i + 1; j < kWeights; ++j) v -= m[j] * sol[j];
+                sol[i] = readlane_f64(v / m[i], order[i]);
+                if (lane == i) mine = sol[i];
+            }
+            ok = __ballot(lane < kWeights && !isfinite(mine)) == 0;
+        }
     }
-    double *w = weights + r * 24;
-    int32_t *q = quantised + r * 24;
+    uint32_t shift = 6;
+    for (uint32_t cand = 9; cand >= 7; --cand) {
+        const double v = round(mine * (double)(1u << cand));
+        if (__ballot(lane < kWeights && !(v >= -128.0 && v <= 127.0)) == 0) {
+            shift = cand;
+            break;
+        }
+    }
+    if (lane < kWeights) {
+        const double v = ok ? fmin(fmax(round(mine * (double)(1u << shift)), -128.0), 127.0) : 0.0;
+        weights[r * kWeights + lane] = ok ? mine : 0.0;
+        quantised[r * kWeights + lane] = (int32_t)v;
+    }
     if (lane == 0) {
-        bool ok = s_ok != 0;
-        if (ok) {
-            for (int i = 23; i >= 0; --i) {
-                double v = s_m[i][24];
-                for (int j = i + 1; j < 24; ++j) v -= s_m[i][j] * s_sol[j];
-                s_sol[i] = v / s_m[i][i];
-            }
-            for (int i = 0; i < 24; ++i) ok = ok && isfinite(s_sol[i]);
-        }
-        uint32_t shift = 6;
-        if (ok) {
-            for (uint32_t cand = 9; cand >= 7; --cand) {
-                bool fits = true;
-                for (int i = 0; i < 24; ++i) {
-                    const double v = round(s_sol[i] * (double)(1u << cand));
-                    fits = fits && v >= -128.0 && v <= 127.0;
-                }
-                if (fits) {
-                    shift = cand;
-                    break;
-                }
-            }
-        }
-        for (int i = 0; i < 24; ++i) {
-            const double v = ok ? fmin(fmax(round(s_sol[i] * (double)(1u << shift)), -128.0), 127.0) : 0.0;
-            w[i] = ok ? s_sol[i] : 0.0;
-            q[i] = (int32_t)v;
-        }
         shifts[r] = ok ? shift : 0u;
         solved[r] = ok ? 1 : 0;
     }
