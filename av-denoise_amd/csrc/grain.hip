@@ -1,46 +1,65 @@
 // Film-grain measurement (grain_measure, nl4d/kernels/grain.rs:243-513; constants
 // nl4d/grain/consts.rs:1-45).
 //
-// One wave per 8x8 cell of channel `channel` at a time, lane l on pixel (l % 8, l / 8); a workgroup
-// of four waves walks 64 consecutive cells, the four waves on neighbouring cells.  Source grain is
-// the motion-compensated difference of ring slots slot_next and slot_t over sqrt 2; one-frame grain
-// is the high-pass std of slot_t over the cell.  A cell that
-// passes the flatness, band, clipping, interior, confidence and std gates adds one count to its
-// brightness bin and std bucket of the source histogram (i32 atomics); a usable cell adds one to
-// the one-frame histogram.  Every cell writes its partial: the 46 lag sums of its mean-free source
-// grain over the cell and a halo of 6 columns each side and 3 rows below (zeros when rejected), its
-// pixel count and its strength group.  Every f32 sum follows the reference's order: the cell sums
-// are 64-slot halving trees (wave shuffles pair the same slots), each lag sum adds the 64 pixels row
-// by row; so the histograms and partials are bit-identical to the reference's.
+// Source grain is the motion-compensated difference of ring slots slot_next and slot_t over sqrt 2;
+// one-frame grain is the high-pass std of slot_t over the 8x8 cell.  A cell that passes the flatness,
+// band, clipping, interior, confidence and std gates adds one count to its brightness bin and std
+// bucket of the source histogram (i32 atomics); a usable cell adds one to the one-frame histogram.
+// Every cell writes its partial: the 46 lag sums of its mean-free source grain over the cell and a halo
+// of 6 columns each side and 3 rows below (zeros when rejected), its pixel count and its strength group.
+// Every f32 sum follows the reference's order: the cell sums are 64-slot halving trees, each lag sum
+// adds the 64 pixels row by row; so the histograms and partials are bit-identical to the reference's.
+//
+// Lanes are columns: eight lanes hold a cell, a wave eight cells side by side, each lane its column's
+// eight rows in registers, so a row is one coalesced load, the tree's three upper levels are adds of
+// registers and its three lower ones DPP adds within eight lanes.
 
 #include "common.h"
 
 namespace avd {
 namespace {
 
-constexpr int kCell = 8, kTileW = 20, kTileH = 11, kHalo = 6, kLags = 46, kPartial = 48;
+constexpr int kCell = 8, kHalo = 6, kHaloRows = 3, kLags = 46, kPartial = 48;
 constexpr int kBuckets = 64, kBins = 16, kHist = kBins * kBuckets;
-constexpr int kWaves = 4, kCellsPerGroup = 64;  // 16 cells per wave
+// A measuring workgroup's cells: a wave takes eight of a row.
+constexpr int kGroupX = 16, kGroupY = 2, kMeasureThreads = kGroupX * kGroupY * kCell;
+constexpr int kPlaneW = kGroupX * kCell + 2 * kHalo, kPlaneH = kGroupY * kCell + kHaloRows;
 
-__device__ inline float tree64(float v)
+template <int CTRL>
+__device__ __forceinline__ float dpp(float v)
 {
-#pragma unroll
-    for (int stride = 32; stride >= 1; stride >>= 1) v += __shfl_down(v, stride);
-    return __shfl(v, 0);
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xf, 0xf, true));
 }
 
-__device__ inline float min64(float v)
+// Lane l ^ 4, l ^ 2, l ^ 1 in turn: the lower levels of a cell's halving tree, whose total reaches all
+// eight lanes (an add is the same both ways round).
+__device__ __forceinline__ float sum8(float v)
 {
-#pragma unroll
-    for (int stride = 32; stride >= 1; stride >>= 1) v = fminf(v, __shfl_xor(v, stride));
+    v += dpp<0x141>(dpp<0x1B>(v));  // row_half_mirror of quad_perm 3,2,1,0
+    v += dpp<0x4E>(v);              // quad_perm 2,3,0,1
+    v += dpp<0xB1>(v);              // quad_perm 1,0,3,2
     return v;
 }
 
-__device__ inline float max64(float v)
+__device__ __forceinline__ float min8(float v)
 {
-#pragma unroll
-    for (int stride = 32; stride >= 1; stride >>= 1) v = fmaxf(v, __shfl_xor(v, stride));
-    return v;
+    v = fminf(v, dpp<0x141>(v));
+    v = fminf(v, dpp<0x4E>(v));
+    return fminf(v, dpp<0xB1>(v));
+}
+
+__device__ __forceinline__ float max8(float v)
+{
+    v = fmaxf(v, dpp<0x141>(v));
+    v = fmaxf(v, dpp<0x4E>(v));
+    return fmaxf(v, dpp<0xB1>(v));
+}
+
+// The cell's 64-slot halving tree: a slot is row * 8 + column, so strides 32, 16 and 8 pair rows.
+template <class F>
+__device__ __forceinline__ float tree_cell(F row)
+{
+    return sum8(((row(0) + row(4)) + (row(2) + row(6))) + ((row(1) + row(5)) + (row(3) + row(7))));
 }
 
 // Rust's saturating float-to-u32 cast, for the brightness bins.
@@ -53,17 +72,29 @@ __device__ inline uint32_t block_for(int cx, int cy, uint32_t bx, uint32_t by, u
     return min((uint32_t)(cx * kCell) / step, bx - 1) + min((uint32_t)(cy * kCell) / step, by - 1) * bx;
 }
 
-// The highest bucket whose lower edge is at or below s (bucket_for, grain.rs:193-205).
-__device__ inline uint32_t bucket_for(float s, const float *edges)
+// The highest bucket whose lower edge is at or below s (bucket_for, grain.rs:193-205): lane lx of the
+// cell holds the edges of buckets 8 lx to 8 lx + 7.
+__device__ inline uint32_t bucket_for(float s, const float (&edge)[kBuckets / 8], int lx)
 {
-    uint32_t b = 0;
-    for (uint32_t i = 1; i < kBuckets; ++i) b = s >= edges[i] ? i : b;
-    return b;
+    int b = 0;
+#pragma unroll
+    for (int j = 0; j < kBuckets / 8; ++j) b = s >= edge[j] ? lx * (kBuckets / 8) + j : b;
+    b = max(b, __builtin_amdgcn_update_dpp(0, b, 0x141, 0xf, 0xf, true));
+    b = max(b, __builtin_amdgcn_update_dpp(0, b, 0x4E, 0xf, 0xf, true));
+    b = max(b, __builtin_amdgcn_update_dpp(0, b, 0xB1, 0xf, 0xf, true));
+    return (uint32_t)b;
 }
 
 __device__ inline uint32_t luma_bin(float mean) { return min(sat_u32(mean * (float)kBins), (uint32_t)kBins - 1); }
 
-__global__ __launch_bounds__(64 * kWaves) void k_grain_measure(
+// A workgroup of four waves takes 16 x 2 cells.  An accepted cell is an interior one, so its halo lies in
+// whole cells and holds those cells' own grain: the workgroup keeps one plane of grain in LDS, its own
+// pixels and a rim, and no pixel is fetched per cell.  In the lag sums lane lx of a cell takes six or
+// seven neighbouring lags of one row offset, whose windows share their fourteen plane values.
+// Bound by VALU issue (the lag sums' ordered multiplies and adds are half of it) and the chain vector ->
+// sample -> tree -> lags.  1920x1080, one wave per cell with shuffle trees, a lane per lag and 156 halo
+// pixels fetched per cell: 120 us; this form 17 us.
+__global__ __launch_bounds__(kMeasureThreads) void k_grain_measure(
     const float *__restrict__ ring, const float *__restrict__ out_t, const int32_t *__restrict__ saved_mv,
     const float *__restrict__ saved_conf, const float *__restrict__ edges, const float *__restrict__ luma_means,
     int *__restrict__ hist, float *__restrict__ partials, int W, int H, int C, int ch, uint32_t slot_t,
@@ -73,200 +104,229 @@ __global__ __launch_bounds__(64 * kWaves) void k_grain_measure(
     // The workgroup's counts gather in LDS and reach `hist` as one atomic per non-empty bin: a flat
     // region sends every cell to the same bin, where per-cell global atomics would serialise.
     __shared__ int s_hist[2 * kHist];
-    __shared__ float s_tile[kWaves][kTileW * kTileH];
-    const int t = (int)threadIdx.x, lane = t & 63, wave = t >> 6;
-    for (int i = t; i < 2 * kHist; i += 64 * kWaves) s_hist[i] = 0;
-    __syncthreads();
-
-    const int cells_x = W / kCell, cells_y = H / kCell, cells = cells_x * cells_y;
-    const int lx = lane & 7, ly = lane >> 3;
-    const size_t plane = (size_t)W * H;
+    __shared__ int2 s_vec[kGroupY + 1][kGroupX + 2];  // the group's cells', the rim's cells' vectors
+    __shared__ __align__(16) float s_grain[kPlaneH * kPlaneW];
+    __shared__ __align__(16) float s_centre[kGroupY * kCell][kGroupX * kCell];  // mean-free
+    const int t = (int)threadIdx.x, lane = t & 63, wave = t >> 6, lx = lane & 7;
+    const int cells_x = W / kCell, cells_y = H / kCell;
+    const int gx = (int)blockIdx.x * kGroupX, gy = (int)blockIdx.y * kGroupY;
+    const int tcx = (wave & 1) * 8 + (lane >> 3), tcy = wave >> 1;  // the lane's cell in the group
+    const bool live = gx + tcx < cells_x && gy + tcy < cells_y;
+    const int cx = min(gx + tcx, cells_x - 1), cy = min(gy + tcy, cells_y - 1);
+    const int x = cx * kCell + lx, oy = cy * kCell;
+    const size_t plane = (size_t)W * H, row_len = (size_t)W * C;
     const float *ft = ring + (size_t)slot_t * plane * C + ch, *fnx = ring + (size_t)slot_next * plane * C + ch;
     const uint32_t blocks = bx * by, base = entry * blocks * 2;
     constexpr float kR2 = 0.70710677f;
-    float *tile = s_tile[wave];
 
-    // Wave w takes cells first + w, first + w + 4, ...: the four waves work on neighbouring cells.
-    const int first = (int)blockIdx.x * kCellsPerGroup;
-    for (int k = 0; k < kCellsPerGroup / kWaves; ++k) {
-        const int cell = first + wave + k * kWaves;
-        if (cell >= cells) break;  // uniform per wave; only the final barrier follows the loop
-        // The previous cell's lag sums have read the tile.
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        const int cx = cell % cells_x, cy = cell / cells_x, ox = cx * kCell, oy = cy * kCell;
-        const int x = ox + lx, y = oy + ly;
-        const uint32_t blk = block_for(cx, cy, bx, by, step);
-        const int dx = saved_mv[base + blk * 2], dy = saved_mv[base + blk * 2 + 1];
-
-        const float cur = ft[((size_t)y * W + x) * C];
-        const float nxt = fnx[((size_t)shift_clamp(y, dy, H) * W + shift_clamp(x, dx, W)) * C];
-        const float g = (nxt - cur) * kR2;
-        const float clean = out_t[((size_t)y * W + x) * C + ch];
-        const float origin = ft[((size_t)oy * W + ox) * C];
-        tile[ly * kTileW + lx + kHalo] = g;
-
-        // One-frame high pass (neighbour_squares, grain.rs:251-269): squared steps to the right and
-        // lower neighbours inside the cell, relative to the origin sample.
-        const float fv = cur - origin;
-        const float right = __shfl_down(fv, 1), down = __shfl_down(fv, 8);
-        float hp = 0.0f;
-        if (lx + 1 < kCell) hp += (right - fv) * (right - fv);
-        if (ly + 1 < kCell) hp += (down - fv) * (down - fv);
-
-        const float sum = tree64(g), sum_sq = tree64(g * g), clean_sum = tree64(clean), hp_sum = tree64(hp);
-        const float clean_lo = min64(clean), clean_hi = max64(clean);
-        const float src_lo = min64(fminf(cur, nxt)), src_hi = max64(fmaxf(cur, nxt));
-
-        const float count = 64.0f;
-        const float var = (sum_sq - sum * sum / count) / (count - 1.0f);
-        const float grain_std = sqrtf(fmaxf(var, 0.0f));
-        const float mean = clean_sum / count;
-        const float frame_std = sqrtf(hp_sum / 224.0f);
-        const float range = clean_hi - clean_lo;
-        const bool interior = cx >= 1 && cx + 2 <= cells_x && cy + 2 <= cells_y;
-        const float conf = saved_conf[entry * blocks + blk];
-        const bool band = !luma_band || (mean > 20.0f / 255.0f && mean < 235.0f / 255.0f);
-        const bool usable = has_source && range < 5.0f / 255.0f && band && src_lo >= 4.0f / 255.0f &&
-                            src_hi <= 251.0f / 255.0f;
-        const bool passes = usable && interior && conf >= 0.8f && grain_std > 0.05f / 255.0f;
-        const bool frame_passes = usable && (means_bx == 0 || has_luma_means);
-        uint32_t group = 0;
-        if (passes) {
-            const uint32_t b = bucket_for(grain_std, edges);
-            group = b / 4;
-            if (lane == 0) atomicAdd(s_hist + luma_bin(mean) * kBuckets + b, 1);
-        }
-        if (frame_passes && lane == 0) {
-            const uint32_t b = bucket_for(frame_std, edges);
-            uint32_t bin = luma_bin(mean);
-            if (means_bx > 0) {
-                const uint32_t mb = (uint32_t)(cy * kCell / 16) * means_bx + (uint32_t)(cx * kCell / 16);
-                bin = min(sat_u32(luma_means[mb * 3] / 16.0f), (uint32_t)kBins - 1);
-            }
-            atomicAdd(s_hist + kHist + bin * kBuckets + b, 1);
-        }
-
-        // The accepted cell's halo of source grain, each pixel with its own cell's vector, clamped
-        // into the frame (grain.rs:441-475).  Four unrolled steps: every vector load goes out, then
-        // every sample load.
-        if (passes) {
-            constexpr int kSteps = (kTileW * kTileH + 63) / 64;
-            int hx[kSteps], hy[kSteps], ex[kSteps], ey[kSteps];
-            bool halo[kSteps];
+    float cur[kCell], clean[kCell];
+    {
+        const size_t at = ((size_t)oy * W + x) * C;
 #pragma unroll
-            for (int j = 0; j < kSteps; ++j) {
-                const int f = lane + 64 * j, tx = f % kTileW, ty = f / kTileW;
-                halo[j] = f < kTileW * kTileH && !(ty < kCell && tx >= kHalo && tx < kHalo + kCell);
-                hx[j] = shift_clamp(0, ox + tx - kHalo, W);
-                hy[j] = shift_clamp(oy + min(ty, kTileH - 1), 0, H);
-                const uint32_t b2 = block_for(hx[j] / kCell, hy[j] / kCell, bx, by, step);
-                ex[j] = saved_mv[base + b2 * 2];
-                ey[j] = saved_mv[base + b2 * 2 + 1];
-            }
-            float vn[kSteps], vt[kSteps];
-#pragma unroll
-            for (int j = 0; j < kSteps; ++j) {
-                vn[j] = fnx[((size_t)shift_clamp(hy[j], ey[j], H) * W + shift_clamp(hx[j], ex[j], W)) * C];
-                vt[j] = ft[((size_t)hy[j] * W + hx[j]) * C];
-            }
-#pragma unroll
-            for (int j = 0; j < kSteps; ++j)
-                if (halo[j]) tile[lane + 64 * j] = (vn[j] - vt[j]) * kR2;
-        }
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-
-        float *part = partials + (size_t)cell * kPartial;
-        if (lane < kLags) {
-            // Lane l sums lag l (dy 0: dx 0..6; dy 1..3: dx -6..6) over the cell's pixels in row order.
-            const int row = lane > kHalo ? 1 + (lane - kHalo - 1) / 13 : 0;
-            const int col = lane > kHalo ? (lane - kHalo - 1) % 13 : lane + kHalo;
-            const float gmean = sum / 64.0f;
-            float acc = 0.0f;
-            if (passes) {
-#pragma unroll 16
-                for (int p = 0; p < 64; ++p) {
-                    const int px = p & 7, py = p >> 3;
-                    const float c = tile[py * kTileW + px + kHalo] - gmean;
-                    const float n = tile[(py + row) * kTileW + px + col] - gmean;
-                    acc += c * n;
-                }
-            }
-            part[lane] = acc;
-        } else if (lane == kLags) {
-            part[kLags] = passes ? 64.0f : 0.0f;
-        } else if (lane == kLags + 1) {
-            part[kLags + 1] = (float)group;
+        for (int r = 0; r < kCell; ++r) {
+            cur[r] = ft[at + r * row_len];
+            clean[r] = out_t[at + r * row_len + ch];
         }
     }
-
+    const float conf = saved_conf[entry * blocks + block_for(cx, cy, bx, by, step)];
+    float edge[kBuckets / 8] = {};
+    if (has_source) {
+#pragma unroll
+        for (int j = 0; j < kBuckets / 8; ++j) edge[j] = edges[max(lx * (kBuckets / 8) + j, 1)];
+    }
+    for (int i = t; i < 2 * kHist / 4; i += kMeasureThreads) ((int4 *)s_hist)[i] = make_int4(0, 0, 0, 0);
+    if (t < (kGroupY + 1) * (kGroupX + 2)) {
+        const int vx = min(max(gx - 1 + t % (kGroupX + 2), 0), cells_x - 1);
+        const int vy = min(gy + t / (kGroupX + 2), cells_y - 1);
+        const uint32_t b = base + block_for(vx, vy, bx, by, step) * 2;
+        s_vec[t / (kGroupX + 2)][t % (kGroupX + 2)] = make_int2(saved_mv[b], saved_mv[b + 1]);
+    }
     __syncthreads();
-    for (int i = t; i < 2 * kHist; i += 64 * kWaves) {
+
+    float nxt[kCell];
+    {
+        const int2 v = s_vec[tcy][tcx + 1];
+        const float *column = fnx + (size_t)shift_clamp(x, v.x, W) * C;
+#pragma unroll
+        for (int r = 0; r < kCell; ++r) nxt[r] = column[shift_clamp(oy + r, v.y, H) * row_len];
+    }
+    // The rim: three rows below the group, then six columns on either side of all rows.  A pixel past
+    // the last whole cell takes the nearest one's, which no accepted cell reads.
+    constexpr int kBelow = kHaloRows * kGroupX * kCell, kRim = kBelow + 2 * kHalo * kPlaneH;
+    constexpr int kRimSteps = (kRim + kMeasureThreads - 1) / kMeasureThreads;
+    float rim[kRimSteps];
+#pragma unroll
+    for (int j = 0; j < kRimSteps; ++j) {
+        const int f = t + kMeasureThreads * j, side = f - kBelow;
+        const int ty = side < 0 ? kGroupY * kCell + f / (kGroupX * kCell) : min(side / (2 * kHalo), kPlaneH - 1);
+        const int sx = side % (2 * kHalo);
+        const int tx = side < 0 ? kHalo + f % (kGroupX * kCell) : sx < kHalo ? sx : sx + kGroupX * kCell;
+        const int hx = min(max(gx * kCell + tx - kHalo, 0), cells_x * kCell - 1);
+        const int hy = min(gy * kCell + ty, cells_y * kCell - 1);
+        const int2 v = s_vec[hy / kCell - gy][hx / kCell - gx + 1];
+        const float n = fnx[((size_t)shift_clamp(hy, v.y, H) * W + shift_clamp(hx, v.x, W)) * C];
+        rim[j] = (n - ft[((size_t)hy * W + hx) * C]) * kR2;
+        if (f < kRim) s_grain[ty * kPlaneW + tx] = rim[j];
+    }
+
+    float g[kCell];
+#pragma unroll
+    for (int r = 0; r < kCell; ++r) {
+        g[r] = (nxt[r] - cur[r]) * kR2;
+        s_grain[(tcy * kCell + r) * kPlaneW + kHalo + tcx * kCell + lx] = g[r];
+    }
+    // One-frame high pass (neighbour_squares, grain.rs:251-269): squared steps to the right and lower
+    // neighbours inside the cell, relative to the origin sample.
+    const float origin = __shfl(cur[0], lane & ~7);
+    float fv[kCell], hp[kCell];
+#pragma unroll
+    for (int r = 0; r < kCell; ++r) fv[r] = cur[r] - origin;
+#pragma unroll
+    for (int r = 0; r < kCell; ++r) {
+        const float right = dpp<0x101>(fv[r]) - fv[r];  // row_shl 1: the next lane
+        hp[r] = lx + 1 < kCell ? right * right : 0.0f;
+        if (r + 1 < kCell) hp[r] += (fv[r + 1] - fv[r]) * (fv[r + 1] - fv[r]);
+    }
+
+    const float sum = tree_cell([&](int r) { return g[r]; }), sum_sq = tree_cell([&](int r) { return g[r] * g[r]; });
+    const float clean_sum = tree_cell([&](int r) { return clean[r]; }), hp_sum = tree_cell([&](int r) { return hp[r]; });
+    float clean_lo = clean[0], clean_hi = clean[0], src_lo = fminf(cur[0], nxt[0]), src_hi = fmaxf(cur[0], nxt[0]);
+#pragma unroll
+    for (int r = 1; r < kCell; ++r) {
+        clean_lo = fminf(clean_lo, clean[r]);
+        clean_hi = fmaxf(clean_hi, clean[r]);
+        src_lo = fminf(src_lo, fminf(cur[r], nxt[r]));
+        src_hi = fmaxf(src_hi, fmaxf(cur[r], nxt[r]));
+    }
+    clean_lo = min8(clean_lo);
+    clean_hi = max8(clean_hi);
+    src_lo = min8(src_lo);
+    src_hi = max8(src_hi);
+
+    const float count = 64.0f;
+    const float var = (sum_sq - sum * sum / count) / (count - 1.0f);
+    const float grain_std = sqrtf(fmaxf(var, 0.0f));
+    const float mean = clean_sum / count;
+    const float frame_std = sqrtf(hp_sum / 224.0f);
+    const float range = clean_hi - clean_lo;
+    const bool interior = cx >= 1 && cx + 2 <= cells_x && cy + 2 <= cells_y;
+    const bool band = !luma_band || (mean > 20.0f / 255.0f && mean < 235.0f / 255.0f);
+    const bool usable = live && has_source && range < 5.0f / 255.0f && band && src_lo >= 4.0f / 255.0f &&
+                        src_hi <= 251.0f / 255.0f;
+    const bool passes = usable && interior && conf >= 0.8f && grain_std > 0.05f / 255.0f;
+    const bool frame_passes = usable && (means_bx == 0 || has_luma_means);
+    // Whole waves look the buckets up together: their eight lanes exchange.
+    const uint32_t bucket = bucket_for(grain_std, edge, lx), frame_bucket = bucket_for(frame_std, edge, lx);
+    if (lx == 0 && passes) atomicAdd(s_hist + luma_bin(mean) * kBuckets + bucket, 1);
+    if (lx == 0 && frame_passes) {
+        uint32_t bin = luma_bin(mean);
+        if (means_bx > 0) {
+            const uint32_t mb = (uint32_t)(cy * kCell / 16) * means_bx + (uint32_t)(cx * kCell / 16);
+            bin = min(sat_u32(luma_means[mb * 3] / 16.0f), (uint32_t)kBins - 1);
+        }
+        atomicAdd(s_hist + kHist + bin * kBuckets + frame_bucket, 1);
+    }
+    const float gmean = sum / 64.0f;
+#pragma unroll
+    for (int r = 0; r < kCell; ++r) s_centre[tcy * kCell + r][tcx * kCell + lx] = g[r] - gmean;
+    __syncthreads();
+
+    // Lane lx takes the lags of row offset `row` from plane column `col` on: dy 0's seven, then six and
+    // seven of each further row; lane 7 writes the count and the group.
+    constexpr int kRun = 7;
+    const int role = min(lx, 6), row = (role + 1) >> 1, col = role & 1 ? 0 : kHalo;
+    float acc[kRun];
+#pragma unroll
+    for (int k = 0; k < kRun; ++k) acc[k] = 0.0f;
+    if (__any(passes)) {
+        const float *c_at = &s_centre[tcy * kCell][tcx * kCell];
+        const float *n_at = s_grain + (tcy * kCell + row) * kPlaneW + tcx * kCell + col;
+#pragma unroll 1
+        for (int py = 0; py < kCell; ++py, c_at += kGroupX * kCell, n_at += kPlaneW) {
+            float c[kCell], n[kCell + kRun - 1];
+#pragma unroll
+            for (int i = 0; i < kCell / 4; ++i) *(float4 *)(c + 4 * i) = ((const float4 *)c_at)[i];
+#pragma unroll
+            for (int i = 0; i < (kCell + kRun - 1) / 2; ++i) *(float2 *)(n + 2 * i) = ((const float2 *)n_at)[i];
+#pragma unroll
+            for (int i = 0; i < kCell + kRun - 1; ++i) n[i] -= gmean;
+#pragma unroll
+            for (int px = 0; px < kCell; ++px)
+#pragma unroll
+                for (int k = 0; k < kRun; ++k) acc[k] += c[px] * n[px + k];
+        }
+    }
+    if (lx == 7) {
+        acc[0] = 64.0f;
+        acc[1] = (float)(bucket / 4);
+    }
+    if (live) {
+        float *part = partials + ((size_t)cy * cells_x + cx) * kPartial;
+        part += lx == 7 ? kLags : row == 0 ? 0 : kRun + (row - 1) * 13 + col;
+#pragma unroll
+        for (int k = 0; k < kRun; ++k)
+            if (k < (lx == 7 ? 2 : col == 0 ? kRun - 1 : kRun)) part[k] = passes ? acc[k] : 0.0f;
+    }
+
+    for (int i = t; i < 2 * kHist; i += kMeasureThreads) {
         const int n = s_hist[i];
         if (n) atomicAdd(hist + i, n);
     }
 }
 
-// grain_reduce_partials (grain.rs:515-560): workgroup `lane` of 47 takes one record lane; thread t
-// of 128 adds lane `lane` of cells t, t + 128, ... in turn into its strength group's column (the
-// group clamped to 15), then each group's 128 columns fold by a halving tree (the 64-stride step
-// through LDS, the rest as wave shuffles, the same slot pairs) and group g's total is added into
-// chunk[record_offset + 47 g + lane].  The 16 columns of a thread stay in registers: each cell adds
-// its value to its own group's and an exact +0.0 to the others (a column starts at +0.0 and so
-// never holds -0.0, which an added +0.0 would change), keeping the reference's order without an LDS
-// read-modify-write on the chain.
+// grain_reduce_partials (grain.rs:515-560): for each record lane, column t of 128 adds the lane of
+// cells t, t + 128, ... in turn into its strength group's sum (the group clamped to 15), then each
+// group's 128 columns fold by a halving tree (the 64-stride step through LDS, the rest as wave shuffles,
+// the same slot pairs) and group g's total is added into chunk[record_offset + 47 g + lane].
+//
+// Workgroup (s, g) takes record lanes 16 s to 16 s + 15 of group g: four threads a column, four lanes a
+// thread.  A cell of another group adds an exact +0.0 (a column starts at +0.0 and so never holds -0.0,
+// which an added +0.0 would change).  The ordered columns keep a total in one workgroup, so the bound is
+// one compute unit's fill rate: the lanes and the group of a cell lie in different cache lines.  32400
+// cells: a workgroup per lane, a column's 16 groups in one thread, 61 us; four lanes of a group per
+// workgroup 57 to 59; two groups in sixteen lanes 60; this split 50 to 52.
 constexpr int kReduceThreads = 128, kGroups = 16, kRecordLen = kLags + 1;
+constexpr int kSector = 16, kSectors = kPartial / kSector;
 
-__global__ __launch_bounds__(kReduceThreads) void k_grain_reduce(const float *__restrict__ partials,
-                                                                 float *__restrict__ chunk, uint32_t record_offset,
-                                                                 uint32_t cells)
+__global__ __launch_bounds__(4 * kReduceThreads) void k_grain_reduce(const float *__restrict__ partials,
+                                                                     float *__restrict__ chunk,
+                                                                     uint32_t record_offset, uint32_t cells)
 {
-    __shared__ float s_col[kGroups][kReduceThreads];
-    const uint32_t lane = blockIdx.x, t = threadIdx.x;
-    float acc[kGroups];
-#pragma unroll
-    for (int g = 0; g < kGroups; ++g) acc[g] = 0.0f;
-    auto add = [&](float v, float gv) {
-        const uint32_t group = min(sat_u32(gv), (uint32_t)kGroups - 1);
-#pragma unroll
-        for (int g = 0; g < kGroups; ++g) acc[g] += group == (uint32_t)g ? v : 0.0f;
+    struct __attribute__((aligned(4))) Quad {  // the caller's floats: a single float's alignment
+        float v[4];
     };
+    __shared__ float s_col[kSector][kReduceThreads + 1];
+    const uint32_t group = blockIdx.y, t = threadIdx.x >> 2, quad = threadIdx.x & 3;
+    const float *part = partials + blockIdx.x * kSector + quad * 4, *groups = partials + kLags + 1;
+    float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
     constexpr uint32_t kBatch = 8;
-    uint32_t c = t;
-    for (; c + (kBatch - 1) * kReduceThreads < cells; c += kBatch * kReduceThreads) {
-        float v[kBatch], gv[kBatch];
+    for (uint32_t c = t; c < cells; c += kBatch * kReduceThreads) {
+        Quad v[kBatch];
+        float gv[kBatch];
 #pragma unroll
         for (uint32_t j = 0; j < kBatch; ++j) {
-            const size_t at = (size_t)(c + j * kReduceThreads) * kPartial;
-            v[j] = partials[at + lane];
-            gv[j] = partials[at + kLags + 1];
+            const size_t at = (size_t)min(c + j * kReduceThreads, cells - 1) * kPartial;
+            v[j] = *(const Quad *)(part + at);
+            gv[j] = groups[at];
         }
 #pragma unroll
-        for (uint32_t j = 0; j < kBatch; ++j) add(v[j], gv[j]);
-    }
-    for (; c < cells; c += kReduceThreads) {
-        const size_t at = (size_t)c * kPartial;
-        add(partials[at + lane], partials[at + kLags + 1]);
+        for (uint32_t j = 0; j < kBatch; ++j) {
+            const bool mine = c + j * kReduceThreads < cells && min(sat_u32(gv[j]), (uint32_t)kGroups - 1) == group;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) acc[e] += mine ? v[j].v[e] : 0.0f;
+        }
     }
 #pragma unroll
-    for (int g = 0; g < kGroups; ++g) s_col[g][t] = acc[g];
+    for (int e = 0; e < 4; ++e) s_col[quad * 4 + e][t] = acc[e];
     __syncthreads();
-    if (t < 64) {
-        float total[kGroups];
+    const uint32_t wave = threadIdx.x >> 6, l = threadIdx.x & 63;
 #pragma unroll
-        for (int g = 0; g < kGroups; ++g) {
-            float x = s_col[g][t] + s_col[g][t + 64];
+    for (uint32_t i = wave; i < kSector; i += 4 * kReduceThreads / 64) {
+        float x = s_col[i][l] + s_col[i][l + 64];
 #pragma unroll
-            for (int stride = 32; stride >= 1; stride >>= 1) x += __shfl_down(x, stride);
-            total[g] = x;
-        }
-        if (t == 0) {
-#pragma unroll
-            for (int g = 0; g < kGroups; ++g) chunk[record_offset + g * kRecordLen + lane] += total[g];
-        }
+        for (int stride = 32; stride >= 1; stride >>= 1) x += __shfl_down(x, stride);
+        const uint32_t lane = blockIdx.x * kSector + i;
+        if (l == 0 && lane < kRecordLen) chunk[record_offset + group * kRecordLen + lane] += x;
     }
 }
 
@@ -448,10 +508,11 @@ __global__ void k_grain_save_vectors(const int32_t *__restrict__ mv_field, const
     }
 }
 
-// grain_project (grain_persistence.rs:54-153): one wave per 8x8 cell, four cells per workgroup.  The
-// eight pattern projections (pixel y * 8 + x added where the pattern bit is set, taken away where
-// clear) and the denoised mean are 64-slot shuffle trees, the extremes butterflies; lane 0 writes
-// the cell's history entry (8 projections and the flat flag).
+// grain_project (grain_persistence.rs:54-153): a wave per eight neighbouring cells, eight lanes a cell.
+// The eight pattern projections (pixel y * 8 + x added where the pattern bit is set, taken away where
+// clear) and the denoised mean are the cell's 64-slot trees; lane p of the cell writes projection p of
+// its history entry, lane 0 the flat flag behind them.  Bound by memory latency (two frames read once).
+// 1920x1080, one wave per cell with shuffle trees: 32 us; this form 5.4 us.
 constexpr int kProjections = 8, kEntry = kProjections + 1;
 
 __global__ __launch_bounds__(256) void k_grain_project(const float *__restrict__ ring, const float *__restrict__ out,
@@ -459,28 +520,49 @@ __global__ __launch_bounds__(256) void k_grain_project(const float *__restrict__
                                                        float *__restrict__ history, int W, int H, int C, int ch,
                                                        uint32_t frame_slot, uint32_t history_slot, int luma_band)
 {
-    const int lane = (int)threadIdx.x & 63, cells_x = W / kCell, cells = cells_x * (H / kCell);
-    const int cell = (int)blockIdx.x * 4 + ((int)threadIdx.x >> 6);
-    if (cell >= cells) return;  // a whole wave; the kernel has no barrier
-    const int x = cell % cells_x * kCell + (lane & 7), y = cell / cells_x * kCell + (lane >> 3);
-    const float sample = ring[(((size_t)frame_slot * H + y) * W + x) * C + ch];
-    const float clean = out[((size_t)y * W + x) * C + ch];
-    float proj[kProjections];
+    const int lane = (int)threadIdx.x & 63, lx = lane & 7, cells_x = W / kCell, cells_y = H / kCell;
+    const int gx = (int)blockIdx.x * 8 + (lane >> 3), cy = (int)blockIdx.y * 4 + ((int)threadIdx.x >> 6);
+    if (cy >= cells_y) return;  // a whole wave; the kernel has no barrier
+    const int cx = min(gx, cells_x - 1);
+    const size_t row_len = (size_t)W * C, at = ((size_t)cy * kCell * W + cx * kCell + lx) * C + ch;
+    const float *src = ring + (size_t)frame_slot * H * row_len + at, *den = out + at;
+    float sample[kCell], clean[kCell];
+#pragma unroll
+    for (int r = 0; r < kCell; ++r) {
+        sample[r] = src[r * row_len];
+        clean[r] = den[r * row_len];
+    }
+    float mine = 0.0f;
 #pragma unroll
     for (int p = 0; p < kProjections; ++p) {
-        const uint32_t bit = (patterns[p * 2 + (lane >> 5)] >> (lane & 31)) & 1u;
-        proj[p] = tree64(((float)bit * 2.0f - 1.0f) * sample);
+        // Row r's bit is bit (r % 4) * 8 + lx of word r / 4; a clear bit flips the sample's sign.
+        const uint32_t low = ~patterns[p * 2] >> lx, high = ~patterns[p * 2 + 1] >> lx;
+        const float v = tree_cell([&](int r) {
+            const uint32_t flip = ((r < 4 ? low : high) << (31 - (r & 3) * 8)) & 0x80000000u;
+            return __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, sample[r]) ^ flip);
+        });
+        mine = lx == p ? v : mine;
     }
-    const float clean_sum = tree64(clean);
-    const float clean_lo = min64(clean), clean_hi = max64(clean), src_lo = min64(sample), src_hi = max64(sample);
-    if (lane == 0) {
-        float *e = history + ((size_t)history_slot * cells + cell) * kEntry;
+    const float clean_sum = tree_cell([&](int r) { return clean[r]; });
+    float clean_lo = clean[0], clean_hi = clean[0], src_lo = sample[0], src_hi = sample[0];
 #pragma unroll
-        for (int p = 0; p < kProjections; ++p) e[p] = proj[p];
+    for (int r = 1; r < kCell; ++r) {
+        clean_lo = fminf(clean_lo, clean[r]);
+        clean_hi = fmaxf(clean_hi, clean[r]);
+        src_lo = fminf(src_lo, sample[r]);
+        src_hi = fmaxf(src_hi, sample[r]);
+    }
+    clean_lo = min8(clean_lo);
+    clean_hi = max8(clean_hi);
+    src_lo = min8(src_lo);
+    src_hi = max8(src_hi);
+    if (gx < cells_x) {
         const float mean = clean_sum / 64.0f, range = clean_hi - clean_lo;
         const bool band = !luma_band || (mean > 20.0f / 255.0f && mean < 235.0f / 255.0f);
         const bool flat = range < 5.0f / 255.0f && band && src_lo >= 4.0f / 255.0f && src_hi <= 251.0f / 255.0f;
-        e[kProjections] = flat ? 1.0f : 0.0f;
+        float *e = history + ((size_t)history_slot * cells_x * cells_y + (size_t)cy * cells_x + cx) * kEntry;
+        e[lx] = mine;
+        if (lx == 0) e[kProjections] = flat ? 1.0f : 0.0f;
     }
 }
 
@@ -578,8 +660,8 @@ hipError_t launch_grain_measure(const GrainMeasure &m, hipStream_t s)
 {
     const uint32_t cells = (m.width / kCell) * (m.height / kCell);
     if (cells == 0) return hipSuccess;
-    const uint32_t groups = (cells + kCellsPerGroup - 1) / kCellsPerGroup;
-    k_grain_measure<<<groups, 64 * kWaves, 0, s>>>(
+    const dim3 groups(div_up(m.width / kCell, kGroupX), div_up(m.height / kCell, kGroupY));
+    k_grain_measure<<<groups, kMeasureThreads, 0, s>>>(
         m.ring, m.denoised, m.saved_mv, m.saved_conf, m.edges, m.luma_means, m.hist, m.partials, (int)m.width,
         (int)m.height, (int)m.channels, (int)m.channel, m.slot_t, m.slot_next, m.blocks_x, m.blocks_y, m.step,
         m.source_entry, m.has_source ? 1 : 0, m.has_luma_means ? 1 : 0, m.means_blocks_x, m.luma_band ? 1 : 0);
@@ -590,7 +672,7 @@ hipError_t launch_grain_reduce(const float *partials, uint32_t cells, float *chu
                                hipStream_t s)
 {
     if (!partials || !chunk) return hipErrorInvalidValue;
-    k_grain_reduce<<<kRecordLen, kReduceThreads, 0, s>>>(partials, chunk, record_offset, cells);
+    k_grain_reduce<<<dim3(kSectors, kGroups), 4 * kReduceThreads, 0, s>>>(partials, chunk, record_offset, cells);
     return hipGetLastError();
 }
 
@@ -620,9 +702,9 @@ hipError_t launch_grain_project(const float *ring, const float *out, const uint3
 {
     const uint32_t cells = (width / kCell) * (height / kCell);
     if (cells == 0) return hipSuccess;
-    k_grain_project<<<(cells + 3) / 4, 256, 0, s>>>(ring, out, patterns, history, (int)width, (int)height,
-                                                   (int)channels, (int)channel, frame_slot, history_slot,
-                                                   luma_band ? 1 : 0);
+    k_grain_project<<<dim3(div_up(width / kCell, 8), div_up(height / kCell, 4)), 256, 0, s>>>(
+        ring, out, patterns, history, (int)width, (int)height, (int)channels, (int)channel, frame_slot, history_slot,
+        luma_band ? 1 : 0);
     return hipGetLastError();
 }
 
