@@ -804,69 +804,96 @@ __global__ __launch_bounds__(kWaves * 64) void k_centre_codes(avd_collab_pass p,
 //
 // The cross term <P, B> of every (reference, candidate) pair is a matrix product: the references'
 // patches are rows of A, the candidates' patches columns of B, patch elements the shared K.  With
-// codes below 1024 it is exact on v_mfma_f32_16x16x32_f16: B holds 1024 + code (the f16 bit
-// pattern 0x6400 | code, prepared once per pass), A holds the reference codes split into their
-// high and low five bits, so every product and partial sum is an integer below 2^24 and the fp32
-// accumulation is exact in any order; <P, B> = 32 * C_hi + C_lo - 1024 * sum(P).
+// codes below 1024 it is exact on v_mfma_f32_16x16x32_f16: B holds code - 512 (prepared once per
+// pass), A holds -2 (code - 512), so a product is an even integer of at most 2^19 and the sum of 64
+// of them, an accumulator's most, an even one of at most 2^25: every partial sum is exact in fp32 in
+// any order (two channels use two accumulators).  SSD = |P|^2 + |B|^2 + acc, the energies those of the
+// centred codes too.
 //
 // A wave takes a block of 2 x 4 references (2 grid columns, 4 grid rows).  A's 16 rows are the
-// (reference, half) pairs; B's columns are 16 consecutive candidate columns of one candidate row
-// cy, two tiles covering every column any of the 8 references searches, and the wave walks cy down
-// the union of their row ranges, so the 16 lanes of a k-block read consecutive codes of one frame
-// row.  Lane (n, g) receives rows 4g..4g+3 of each product, both halves of references 2g and 2g+1
-// (grid row g) for candidate column n of the tile, forms their keys and keeps a sorted top KM per
-// reference (KM = 8 or 16 group members); the 16 lanes of a row then merge each reference's lists
-// by DPP.
+// (reference, shift) pairs: the patch at image rows 0 to 7 of the K dimension scores candidate row cy,
+// shifted down one row it scores cy + 1, so nine image rows serve two candidate rows.  B's columns are
+// 16 consecutive candidate columns, two tiles covering every column any of the 8 references searches,
+// and the wave walks cy down the union of their row ranges.  An image row is loaded once: a K step's
+// rows (a group) stay in registers while candidate rows use them, the pairs of rows inside a group
+// being further shifts of A.  Lane (n, g) receives rows 4g..4g+3 of each product, both shifts of
+// references 2g and 2g+1 (grid row g) for its candidate column, forms their keys and keeps a sorted
+// top KL per reference; the 16 lanes of a row then merge each reference's lists by DPP.  The lists
+// move four lanes on after every group: along a vertical edge a reference's best candidates share a
+// column, which so falls to four lists.
 //
 // Keys are (min(d, kKeyCap) << 10 | row-major index) in 32 bits.  A reference whose last chosen
-// key reaches the cap (a distance that large could tie-break differently) is listed and searched
-// again with the exact 64-bit keys of the vector search (k_centre_redo).
+// key reaches the cap (a distance that large could tie-break differently) or whose picks outran a
+// lane's list is noted and searched again with the exact 64-bit keys of the vector search
+// (k_centre_redo).
+//
+// Bound by VALU issue: per key its distance and index (5 or 7 instructions) and the list's insertion
+// (KL), then the merge.  Alone, 3840x2160 with 16 members, one / two channels: with the codes in
+// five-bit halves, a candidate row per product, its four operands loaded anew for each, and eight kept
+// keys per lane 1069 / 353 us, and 44 / 130 us of exact searches; this form 634 / 190 us, and 19 / 4 us.
 // ---------------------------------------------------------------------------------------------
 
 typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
 typedef float float4_t __attribute__((ext_vector_type(4)));
 
 constexpr uint32_t kKeyCap = (1u << 22) - 1u;
-constexpr int kPrepRows = 32;
+constexpr int kPrepRows = 8, kPrepCols = 248;
 
-// The centre frame as f16 patterns of 1024 + code (`plane`, and for one channel `plane_odd`, the
-// same shifted by one code so that an 8-code row starting on an odd code is a 4-byte-aligned read)
-// and the energy sum(code^2) of the 8x8 patch at every position x <= W - 8, y <= H - 8.  Thread x
-// of the grid walks kPrepRows rows, keeping the last 8 rows' energies.
+// The centre frame as f16 of code - 512 (`plane`, and for one channel `plane_odd`, the same shifted by
+// one code so that an 8-code row starting on an odd code is a 4-byte-aligned read) and the energy
+// sum((code - 512)^2) of the 8x8 patch at every position x <= W - 8, y <= H - 8.  A workgroup takes
+// kPrepCols columns of kPrepRows rows: a thread sums its column's squares over eight rows, sliding, and
+// eight columns' sums join through LDS.  Bound by memory latency.  A thread walking 32 rows of eight loads
+// each: 427x241 21 to 22 us (16 workgroups), 3840x2160 34 us; this form 4 to 5 and 31 us.
 template <int C>
 __global__ __launch_bounds__(256) void k_centre_prep(const uint16_t *__restrict__ frame, int W, int H,
                                                      uint16_t *__restrict__ plane, uint16_t *__restrict__ plane_odd,
                                                      uint32_t *__restrict__ energy)
 {
-    const int x = blockIdx.x * 256 + threadIdx.x;
-    const int y0 = blockIdx.y * kPrepRows;
-    if (x >= W) return;
-    const size_t n_codes = (size_t)W * H * C;
-    const int y_end = min(y0 + kPrepRows, H);
-    for (int y = y0; y < y_end; ++y) {
+    constexpr int kRead = kPrepRows + 7, kRun = 8, kRuns = kPrepCols / kRun;
+    __shared__ __align__(16) uint32_t s_col[kPrepRows][kPrepCols + 8];
+    const int t = threadIdx.x, x0 = blockIdx.x * kPrepCols, y0 = blockIdx.y * kPrepRows;
+    const int x = min(x0 + t, W - 1);
+    int v[kRead][C];
 #pragma unroll
-        for (int c = 0; c < C; ++c) {
-            const size_t i = ((size_t)y * W + x) * C + c;
-            plane[i] = (uint16_t)(0x6400u | frame[i]);
-            if (C == 1) plane_odd[i] = (uint16_t)(0x6400u | (i + 1 < n_codes ? frame[i + 1] : 0u));
+    for (int r = 0; r < kRead; ++r)
+#pragma unroll
+        for (int c = 0; c < C; ++c) v[r][c] = (int)frame[((size_t)min(y0 + r, H - 1) * W + x) * C + c] - 512;
+    if (t < kPrepCols && x0 + t < W) {
+#pragma unroll
+        for (int r = 0; r < kPrepRows; ++r) {
+            if (y0 + r >= H) break;
+#pragma unroll
+            for (int c = 0; c < C; ++c) {
+                const size_t i = ((size_t)(y0 + r) * W + x) * C + c;
+                const uint16_t h = __builtin_bit_cast(uint16_t, (_Float16)(float)v[r][c]);
+                plane[i] = h;
+                if (C == 1 && i > 0) plane_odd[i - 1] = h;
+            }
         }
     }
-    if (x > W - 8) return;
-    uint32_t rows[8];
-    uint32_t window = 0;
-    const int last = min(y0 + kPrepRows, H - 7) + 7;  // energy rows y0 .. min(y0 + kPrepRows, H - 7) - 1
-    for (int y = y0; y < last; ++y) {
-        uint32_t e = 0;
+    uint32_t sq[kRead], sum = 0;
 #pragma unroll
-        for (int u = 0; u < 8 * C; ++u) {
-            const uint32_t v = frame[((size_t)y * W + x) * C + u];
-            e += v * v;
-        }
-        const int slot = (y - y0) & 7;
-        if (y - y0 >= 8) window -= rows[slot];
-        rows[slot] = e;
-        window += e;
-        if (y - y0 >= 7) energy[(size_t)(y - 7) * W + x] = window;
+    for (int r = 0; r < kRead; ++r) {
+        sq[r] = 0;
+#pragma unroll
+        for (int c = 0; c < C; ++c) sq[r] += (uint32_t)(v[r][c] * v[r][c]);
+        sum += sq[r];
+        if (r >= 8) sum -= sq[r - 8];
+        if (r >= 7) s_col[r - 7][t] = sum;
+    }
+    __syncthreads();
+    const int row = t / kRuns, run = t - row * kRuns;
+    if (row >= kPrepRows || y0 + row > H - 8) return;
+    uint32_t e[kRun + 8];
+#pragma unroll
+    for (int i = 0; i < (kRun + 8) / 4; ++i) *(uint4 *)(e + 4 * i) = ((const uint4 *)&s_col[row][run * kRun])[i];
+    uint32_t *to = energy + (size_t)(y0 + row) * W + x0 + run * kRun;
+    uint32_t window = ((e[0] + e[1]) + (e[2] + e[3])) + ((e[4] + e[5]) + (e[6] + e[7]));
+#pragma unroll
+    for (int k = 0; k < kRun; ++k) {
+        if (x0 + run * kRun + k <= W - 8) to[k] = window;
+        window += e[k + 8] - e[k];
     }
 }
 
@@ -880,28 +907,16 @@ __device__ __forceinline__ uint32_t row16_min_u32(uint32_t v)
     return v;
 }
 
-// Eight consecutive codes of the f16 plane starting at code `a`, as 4-byte-aligned reads: for one
-// channel an odd start reads the shifted copy, `odd_at` elements past the plane.
-template <int C>
-__device__ __forceinline__ half8_t load_b8(const uint16_t *__restrict__ plane, uint32_t odd_at, uint32_t a)
-{
-    const uint32_t i = (C == 1 && (a & 1u)) ? odd_at + a - 1u : a;
-    const uint32_t *q = reinterpret_cast<const uint32_t *>(plane) + (i >> 1);
-    uint32_t w[4];
-#pragma unroll
-    for (int k = 0; k < 4; ++k) w[k] = q[k];
-    return __builtin_bit_cast(half8_t, w);
-}
-
 template <int C, int KM>
-__global__ __launch_bounds__(kWaves * 64) void k_centre_mfma(avd_collab_pass p, const uint16_t *__restrict__ ring,
+__global__ __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_eu(C == 1 ? 4 : 3))) void k_centre_mfma(avd_collab_pass p, const uint16_t *__restrict__ ring,
                                                              const uint16_t *__restrict__ plane, uint32_t odd_at,
                                                              const uint32_t *__restrict__ energy,
                                                              uint32_t *__restrict__ members,
                                                              uint32_t *__restrict__ redo_list,
                                                              unsigned long long *__restrict__ scored_count)
 {
-    constexpr int KS = 2 * C;  // K steps of 32 patch elements
+    // A K step's 32 elements are GROWS image rows, a group; a candidate row pair spans NG groups.
+    constexpr int GROWS = 4 / C, NG = 8 / GROWS + 1, PER = GROWS / 2, SLOTS = NG + 1;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int n = lane & 15, g = lane >> 4;
     const int W = p.width, H = p.height, maxx = W - 8, maxy = H - 8;
@@ -911,7 +926,7 @@ __global__ __launch_bounds__(kWaves * 64) void k_centre_mfma(avd_collab_pass p, 
     const int blk_raw = xcd_block() * kWaves + wave;
     const bool blk_live = blk_raw < blocks_x * blocks_y;
     const int blk = min(blk_raw, blocks_x * blocks_y - 1);
-    const int by = blk / blocks_x, bx = blk - by * blocks_x;
+    const int by = __builtin_amdgcn_readfirstlane(blk / blocks_x), bx = blk - by * blocks_x;
     const size_t cframe = (size_t)p.centre_slot * ((size_t)W * H * C);
 
     // Reference j = 2q + i of the block sits in grid column 2bx + i and grid row 4by + q (both
@@ -921,35 +936,44 @@ __global__ __launch_bounds__(kWaves * 64) void k_centre_mfma(avd_collab_pass p, 
     auto pos_x = [&](int ix) { return min(ix * step, W - 8); };
     auto pos_y = [&](int iy) { return min(iy * step, H - 8); };
 
-    // ---- A: lane (n, g) holds row n (reference n / 2; its high five bits when n is even) at the
-    // k-block g of every K step: patch row 4s + g (one channel) or half g & 1 of row 2s + g / 2.
-    half8_t A[KS];
+    // A k-block's eight elements: row krow of its group (one channel: all of it, two: the half from
+    // element khalf on).
+    const int krow = C == 1 ? g : g >> 1, khalf = C == 1 ? 0 : 8 * (g & 1);
+
+    // ---- A: lane (n, g) holds row n (reference n / 2, shift n % 2) at the k-block g of every K step,
+    // for each of a group's PER row pairs.
+    half8_t A[PER][NG];
     {
-        const int j = n >> 1;
+        const int j = n >> 1, shift = n & 1;
         const int ax = pos_x(ref_col(j & 1)), ay = pos_y(ref_row(j >> 1));
-        const bool hi = (n & 1) == 0;
 #pragma unroll
-        for (int s = 0; s < KS; ++s) {
-            uint32_t w[4];
-            if (C == 1) {
-                load_row<1>(ring, cframe + (size_t)(ay + 4 * s + g) * W + ax, w);
-            } else {
-                const uint32_t *q = reinterpret_cast<const uint32_t *>(
-                    ring + cframe + ((size_t)(ay + 2 * s + (g >> 1)) * W + ax) * 2 + 8 * (g & 1));
+        for (int v = 0; v < PER; ++v)
 #pragma unroll
-                for (int i = 0; i < 4; ++i) w[i] = q[i];
+            for (int s = 0; s < NG; ++s) {
+                const int r = GROWS * s + krow - shift - 2 * v;
+                const bool in = r >= 0 && r < 8;
+                const int ry = ay + min(max(r, 0), 7);
+                uint32_t w[4];
+                if (C == 1) {
+                    load_row<1>(ring, cframe + (size_t)ry * W + ax, w);
+                } else {
+                    const uint32_t *q =
+                        reinterpret_cast<const uint32_t *>(ring + cframe + ((size_t)ry * W + ax) * 2 + khalf);
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) w[i] = q[i];
+                }
+                // 0x6400 | code is 1024 + code in f16, so -2 x + 3072 is -2 (code - 512), exactly.
+#pragma unroll
+                for (int i = 0; i < 4; ++i) w[i] |= 0x64006400u;
+                const half8_t x = __builtin_bit_cast(half8_t, w);
+                const half8_t a = __builtin_elementwise_fma(x, (half8_t)(_Float16)-2.0f, (half8_t)(_Float16)3072.0f);
+                A[v][s] = in ? a : (half8_t)(_Float16)0.0f;
             }
-#pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                const uint32_t code = (w[e >> 1] >> (16 * (e & 1))) & 0xFFFFu;
-                A[s][e] = (_Float16)(float)(hi ? (code >> 5) : (code & 31u));
-            }
-        }
     }
 
     // ---- the two references whose keys this lane forms: j = 2g + r, grid row g, column r.
-    int rx_[2], ry_[2], left_[2], top_[2], bottom_[2], rw_[2], nlive_[2];
-    uint32_t kc_[2];
+    int left_[2], top_[2], rows_[2], rw_[2], nlive_[2];
+    uint32_t kc_[2], self_[2];
     bool live_[2];
     int ref_[2];
 #pragma unroll
@@ -957,112 +981,150 @@ __global__ __launch_bounds__(kWaves * 64) void k_centre_mfma(avd_collab_pass p, 
         const int ix = ref_col(r), iy = ref_row(g);
         live_[r] = blk_live && 2 * bx + r < refs_x && 4 * by + g < refs_y;
         ref_[r] = iy * refs_x + ix;
-        rx_[r] = pos_x(ix);
-        ry_[r] = pos_y(iy);
-        left_[r] = clampi(rx_[r] - S, 0, maxx);
-        const int right = clampi(rx_[r] + S, 0, maxx);
-        top_[r] = clampi(ry_[r] - S, 0, maxy);
-        bottom_[r] = clampi(ry_[r] + S, 0, maxy);
-        rw_[r] = right - left_[r] + 1;
-        nlive_[r] = rw_[r] * (bottom_[r] - top_[r] + 1);
-        // kc = |P|^2 + 2 * 1024 * sum(P): SSD = kc + |B|^2 - 2 * (32 * C_hi + C_lo).
-        uint32_t e2 = 0, sum = 0;
-#pragma unroll
-        for (int v = 0; v < 8; ++v) {
-            uint32_t w[4 * C];
-            load_row<C>(ring, cframe + ((size_t)(ry_[r] + v) * W + rx_[r]) * C, w);
-            e2 = row_dot<C>(w, w, e2);
-#pragma unroll
-            for (int t = 0; t < 4 * C; ++t) sum = __builtin_amdgcn_udot2(as_u2(w[t]), as_u2(0x00010001u), sum, false);
-        }
-        kc_[r] = e2 + 2048u * sum;
+        const int rx = pos_x(ix), ry = pos_y(iy);
+        left_[r] = clampi(rx - S, 0, maxx);
+        rw_[r] = clampi(rx + S, 0, maxx) - left_[r] + 1;
+        top_[r] = clampi(ry - S, 0, maxy);
+        rows_[r] = clampi(ry + S, 0, maxy) - top_[r] + 1;
+        nlive_[r] = rw_[r] * rows_[r];
+        self_[r] = (uint32_t)((ry - top_[r]) * rw_[r] + rx - left_[r]);
+        kc_[r] = energy[(size_t)ry * W + rx] + 1u;  // a key's distance is SSD + 1
     }
-    // Per tile t and reference r: candidate column cx = cx_base + 16 t + n, whether it is searched,
-    // its offset from the rectangle's left edge and whether it is the reference's own column.  A
-    // column past the frame reads the last one (its keys are dropped).
     const int cx_base = clampi(pos_x(ref_col(0)) - S, 0, maxx);
-    bool colok[2][2], selfcol[2][2];
-    int colidx[2][2];
-    uint32_t ecol[2], bcol[KS][2];
-#pragma unroll
-    for (int t = 0; t < 2; ++t) {
-        const int cx = cx_base + 16 * t + n;
-#pragma unroll
-        for (int r = 0; r < 2; ++r) {
-            colok[t][r] = cx >= left_[r] && cx < left_[r] + rw_[r];
-            selfcol[t][r] = cx == rx_[r];
-            colidx[t][r] = cx - left_[r];
-        }
-        const int lx = min(cx, maxx);
-        ecol[t] = (uint32_t)lx;
-#pragma unroll
-        for (int s = 0; s < KS; ++s)
-            bcol[s][t] = C == 1 ? (uint32_t)((4 * s + g) * W + lx) : (uint32_t)(((2 * s + (g >> 1)) * W + lx) * 2 + 8 * (g & 1));
-    }
     const int cy_lo = clampi(pos_y(ref_row(0)) - S, 0, maxy), cy_hi = clampi(pos_y(ref_row(3)) + S, 0, maxy);
 
-    // Each lane keeps its best KL = 8 keys per reference (and counts the keys it was offered): with
-    // sixteen members a reference's best sixteen rarely crowd one lane's two columns (about 2 % of
-    // references put more than eight there on textured 4K content), and a lane that gave up keys
-    // and runs out of kept ones during the merge sends its reference to the exact search.
-    constexpr int KL = 8;
-    uint32_t L[2][KL], offered[2] = {0u, 0u};
+    // Per tile t and reference r: the candidate column's offset from the rectangle's left edge, ~0 where
+    // it is not searched (which survives the saturating add of the row's offset).  A column past the
+    // frame reads the last one (its keys are dropped).  B's rows start on 4-byte boundaries: for one
+    // channel an odd element reads the shifted copy, `odd_at` elements past the plane; a lane's parity
+    // stays, as its rows move by even numbers, so there it is the last column of the lane's parity
+    // (column 1 of a frame with column 0 alone: its eight codes of the shifted copy end with the row).
+    const int lim = C == 1 ? max(maxx - ((maxx ^ (cx_base + n)) & 1), (cx_base + n) & 1) : maxx;
+    uint32_t col_[2][2], plane_[2], energy_[2];
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+        const int cx = cx_base + n + 16 * t;
+#pragma unroll
+        for (int r = 0; r < 2; ++r) {
+            const uint32_t off = (uint32_t)(cx - left_[r]);
+            col_[t][r] = off < (uint32_t)rw_[r] ? off : ~0u;
+        }
+        const uint32_t lx = (uint32_t)min(cx, lim);
+        const bool odd = C == 1 && (((cy_lo + krow) * W + cx) & 1);
+        plane_[t] = 2u * (lx * C + (uint32_t)khalf + (odd ? odd_at - 1u : 0u));
+        energy_[t] = 4u * lx;
+    }
+
+    // Each lane keeps its best KL keys per reference; a lane whose full list runs out during the merge
+    // sends its reference to the exact search.
+    // Seven: with six a 427x241 frame
+    // of eight members sent a reference there (11 us for the one), an eighth costs a twentieth of the loop.
+    constexpr int KL = 7;
+    uint32_t L[2][KL];
 #pragma unroll
     for (int r = 0; r < 2; ++r)
 #pragma unroll
         for (int i = 0; i < KL; ++i) L[r][i] = ~0u;
-    // The next row's operands load while this row's products and keys are formed (two operand
-    // sets in turn, so no copy waits on a load in flight).  cy <= maxy, so every patch row exists.
-    auto load_row_ops = [&](int cy, half8_t (&B)[KS][2], uint32_t (&eb)[2]) {
-        const uint32_t base = (uint32_t)(cy * W * C);
+
+    typedef uint32_t words4_t __attribute__((ext_vector_type(4), aligned(4)));
+    half8_t B[SLOTS][2];
+    uint32_t e_[2][2][2];  // [step parity][tile][candidate row]
+    // The group from image row `row` on.  Rows past the frame serve candidate rows that are not searched
+    // alone: any row of the same parity does.
+    auto load_group = [&](int row, half8_t (&to)[2]) {
+        const int mine = row + krow, over = max(mine - (H - 1), 0);
+        const uint32_t at = (uint32_t)((mine - ((over + 1) & ~1)) * W * C) * 2u;
 #pragma unroll
-        for (int s = 0; s < KS; ++s)
-#pragma unroll
-            for (int t = 0; t < 2; ++t) B[s][t] = load_b8<C>(plane, odd_at, base + bcol[s][t]);
-#pragma unroll
-        for (int t = 0; t < 2; ++t) eb[t] = energy[(uint32_t)(cy * W) + ecol[t]];
+        for (int t = 0; t < 2; ++t)
+            to[t] = __builtin_bit_cast(half8_t, *reinterpret_cast<const words4_t *>(reinterpret_cast<const char *>(plane) +
+                                                                                    (at + plane_[t])));
     };
-    auto score_row = [&](int cy, const half8_t (&B)[KS][2], const uint32_t (&eb)[2]) {
-        float4_t acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+    auto load_energy = [&](int cy, uint32_t (&to)[2][2]) {
 #pragma unroll
-        for (int s = 0; s < KS; ++s)
-#pragma unroll
-            for (int t = 0; t < 2; ++t) acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A[s], B[s][t], acc[t], 0, 0, 0);
-#pragma unroll
-        for (int r = 0; r < 2; ++r) {
-            const bool rowok = cy >= top_[r] && cy <= bottom_[r];
-            const int rowbase = (cy - top_[r]) * rw_[r];
-            const bool selfrow = cy == ry_[r];
+        for (int i = 0; i < 2; ++i) {
+            uint32_t at = (uint32_t)__builtin_amdgcn_readfirstlane(min(cy + i, maxy) * W * 4);
+            asm volatile("" : "+s"(at));
+            const char *base = reinterpret_cast<const char *>(energy) + at;
 #pragma unroll
             for (int t = 0; t < 2; ++t) {
-                const bool ok = rowok && colok[t][r];
-                const uint32_t cross = ((uint32_t)acc[t][2 * r] << 5) + (uint32_t)acc[t][2 * r + 1];
-                const uint32_t ssd = kc_[r] + eb[t] - 2u * cross;
-                const uint32_t d = (selfrow && selfcol[t][r]) ? 0u : ssd + 1u;
-                const uint32_t key = (min(d, kKeyCap) << 10) | (uint32_t)(rowbase + colidx[t][r]);
-                insert_n_u32<KL>(L[r], key | (ok ? 0u : ~0u));
-                offered[r] += ok ? 1u : 0u;
+                uint32_t lane_at = energy_[t];  // a 32-bit offset from a scalar base, not an address per lane
+                asm volatile("" : "+v"(lane_at));
+                to[t][i] = *reinterpret_cast<const uint32_t *>(base + lane_at);
             }
         }
     };
-    half8_t Bx[KS][2], By[KS][2];
-    uint32_t ex[2], ey[2];
-    load_row_ops(cy_lo, Bx, ex);
-    for (int cy = cy_lo; cy <= cy_hi; cy += 2) {
-        load_row_ops(min(cy + 1, cy_hi), By, ey);
-        score_row(cy, Bx, ex);
-        if (cy + 1 > cy_hi) break;
-        load_row_ops(min(cy + 2, cy_hi), Bx, ex);
-        score_row(cy + 1, By, ey);
+    // One group: PER steps, each the candidate rows cy and cy + 1 of both tiles, while the group NG on
+    // and the next step's energies load.
+    int cy = cy_lo;
+    auto next_group = [&](auto at) {
+        constexpr int slot = decltype(at)::value;
+        load_group(cy + GROWS * NG, B[(slot + NG) % SLOTS]);
+#pragma unroll
+        for (int v = 0; v < PER; ++v) {
+            constexpr bool kPairs = PER == 2;
+            const int now = kPairs ? v : slot & 1;
+            load_energy(cy + 2, e_[now ^ 1]);
+            uint32_t row[2][2];  // the candidate rows' index offsets, ~0 outside the rectangle
+#pragma unroll
+            for (int r = 0; r < 2; ++r)
+#pragma unroll
+                for (int i = 0; i < 2; ++i) {
+                    const uint32_t from = (uint32_t)(cy + i - top_[r]);
+                    row[r][i] = from < (uint32_t)rows_[r] ? from * (uint32_t)rw_[r] : ~0u;
+                }
+#pragma unroll
+            for (int t = 0; t < 2; ++t) {
+                // Two channels: eight patch rows of 16 elements over two accumulators of at most 64
+                // elements, image rows 0 to 3 and 8, and 4 to 7.
+                float4_t acc = {0.f, 0.f, 0.f, 0.f}, second = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int s = 0; s < NG; ++s) {
+                    const half8_t b = B[(slot + s) % SLOTS][t];
+                    if (C == 2 && (s == 2 || s == 3)) second = __builtin_amdgcn_mfma_f32_16x16x32_f16(A[v][s], b, second, 0, 0, 0);
+                    else acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(A[v][s], b, acc, 0, 0, 0);
+                }
+#pragma unroll
+                for (int r = 0; r < 2; ++r)
+#pragma unroll
+                    for (int i = 0; i < 2; ++i) {
+                        uint32_t d = kc_[r] + e_[now][t][i] + (uint32_t)(int)acc[2 * r + i];
+                        if (C == 2) d += (uint32_t)(int)second[2 * r + i];
+                        insert_n_u32<KL>(L[r], (min(d, kKeyCap) << 10) | __builtin_elementwise_add_sat(row[r][i], col_[t][r]));
+                    }
+            }
+            cy += 2;
+        }
+        // The lists move four lanes on.
+#pragma unroll
+        for (int r = 0; r < 2; ++r)
+#pragma unroll
+            for (int i = 0; i < KL; ++i)
+                L[r][i] = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)L[r][i], 0x124, 0xF, 0xF, true);  // row_ror 4
+        return cy <= cy_hi;
+    };
+#pragma unroll
+    for (int s = 0; s < NG; ++s) load_group(cy_lo + GROWS * s, B[s]);
+    load_energy(cy_lo, e_[0]);
+    if (C == 1) {
+        while (next_group(std::integral_constant<int, 0>{}) && next_group(std::integral_constant<int, 1>{}) &&
+               next_group(std::integral_constant<int, 2>{}) && next_group(std::integral_constant<int, 3>{})) {
+        }
+    } else {
+        while (next_group(std::integral_constant<int, 0>{}) && next_group(std::integral_constant<int, 1 % SLOTS>{}) &&
+               next_group(std::integral_constant<int, 2 % SLOTS>{}) && next_group(std::integral_constant<int, 3 % SLOTS>{}) &&
+               next_group(std::integral_constant<int, 4 % SLOTS>{}) && next_group(std::integral_constant<int, 5 % SLOTS>{})) {
+        }
     }
 
-    // ---- merge each reference's 16 lists (one DPP row) into its best KM.
+    // ---- merge each reference's 16 lists (one DPP row) into its best KM, the reference itself first.
     uint32_t word[2] = {0u, 0u};
     bool redo[2];
 #pragma unroll
     for (int r = 0; r < 2; ++r) {
-        const uint32_t inv = (65536u + (uint32_t)rw_[r] - 1u) / (uint32_t)rw_[r];  // idx / rw exact below 1024
+        const bool full = L[r][KL - 1] != ~0u;  // keys may have been given up
+        uint32_t mine = n == 0 ? self_[r] : ~0u;  // this lane's member
         uint32_t last = ~0u;
+        int at = 1;
         bool short_list = false;  // this lane ran out of kept keys while a later pick could need one
 #pragma unroll
         for (int m = 0; m < KM; ++m) {
@@ -1071,15 +1133,23 @@ __global__ __launch_bounds__(kWaves * 64) void k_centre_mfma(avd_collab_pass p, 
             if (best != ~0u) {
                 last = best;
                 const uint32_t idx = best & 1023u;
-                const uint32_t qy = (idx * inv) >> 16, qx = idx - qy * (uint32_t)rw_[r];
-                if (n == m) word[r] = pack_pos_t((uint32_t)left_[r] + qx, (uint32_t)top_[r] + qy, 0);
+                // The reference's own key (its distance is the least there is, but duplicates of it at
+                // lower indices sort before it) has its place already.
+                const bool other = idx != self_[r];
+                if (other && n == at) mine = idx;
+                at += other ? 1 : 0;
                 if (head == best) {
 #pragma unroll
                     for (int i = 0; i < KL - 1; ++i) L[r][i] = L[r][i + 1];
                     L[r][KL - 1] = ~0u;
-                    if (m < KM - 1 && L[r][0] == ~0u && offered[r] > (uint32_t)KL) short_list = true;
+                    if (m < KM - 1 && L[r][0] == ~0u && full) short_list = true;
                 }
             }
+        }
+        if (mine != ~0u) {
+            const uint32_t inv = (65536u + (uint32_t)rw_[r] - 1u) / (uint32_t)rw_[r];  // idx / rw exact below 1024
+            const uint32_t qy = (mine * inv) >> 16, qx = mine - qy * (uint32_t)rw_[r];
+            word[r] = pack_pos_t((uint32_t)left_[r] + qx, (uint32_t)top_[r] + qy, 0);
         }
         // Keys sort by the capped distance; once a chosen one is capped, their order may not be
         // the distances' order.  A lane of the reference's row that ran short leaves the picks
@@ -2767,7 +2837,7 @@ hipError_t launch_centre_km(const avd_collab_pass &p, const uint16_t *codes, uin
             return hipErrorInvalidValue;
         const int W = (int)p.width, H = (int)p.height, st = (int)p.step;
         const uint16_t *frame = codes + (size_t)p.centre_slot * W * H * p.channels;
-        const dim3 pg(div_up(W, 256), div_up(H, kPrepRows));
+        const dim3 pg(div_up(W, kPrepCols), div_up(H, kPrepRows));
         const int refs_x = (W - 8 + st - 1) / st + 1, refs_y = (H - 8 + st - 1) / st + 1;
         const unsigned gm = div_up(((refs_x + 1) / 2) * ((refs_y + 3) / 4), kWaves);
         const hipError_t e = launch_fill_u32(centre->redo, 0, 1, s);

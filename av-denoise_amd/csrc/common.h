@@ -90,9 +90,9 @@ hipError_t launch_map_luma_fields(const FieldMap &m, const int32_t *luma, int32_
 // `scored_count`, when non-null, points at kScoreSlots counters kScoreStride apart; their sum gains
 // the candidate patches the launch scores times the channels.
 constexpr int kScoreSlots = 64, kScoreStride = 16;
-// Scratch of the matrix-core centre search: the centre frame as f16 patterns of 1024 + code
-// (`plane`, W*H*C u16; `plane_odd`, the same shifted by one code, W*H u16, one channel only) and
-// the 8x8 patch energy of every position (`energy`, W*H u32), and the references searched again
+// Scratch of the matrix-core centre search: the centre frame as f16 of code - 512 (`plane`,
+// W*H*C u16; `plane_odd`, the same shifted by one code, W*H u16, one channel only) and the 8x8 patch
+// energy of every position in those (`energy`, W*H u32), and the references searched again
 // with exact keys (`redo`: a count, then the references).
 struct CentreScratch {
     uint16_t *plane, *plane_odd;
