@@ -2551,12 +2551,29 @@ __global__ __launch_bounds__(kWaves * 64) void k_collab_filter_mixed(avd_collab_
     }
 }
 
-// One workgroup per (slot, 32x32 tile): the listed members' positions and group weights are
-// fetched 256 at a time into LDS, then each wave walks members with lane (r, q) on pixel (r, q)
-// of the patch, adding its staged sum and its weight (recomputed from the group weight in the
-// filter's own arithmetic) to the tile in LDS.  The tile then adds to the accumulators once, as
+// round(clamp(w, 0, 1) scale 5) of to_fixed_weight for the gather: the product is not negative, so
+// rounding half away from zero is its truncation plus one where the rest reaches a half (exact: a
+// product of 2^23 or more is whole).
+__device__ __forceinline__ int32_t to_fixed_weight_up(float w, float scale)
+{
+    const float c = fminf(fmaxf(w, 0.0f), 1.0f) * scale * 5.0f;
+    const int32_t i = (int32_t)c;
+    return i + (c - (float)i >= 0.5f ? 1 : 0);
+}
+
+// One workgroup per (slot, 32x32 tile): the listed members' tile cells, ids and group weights are
+// worked out 256 at a time, a thread each, into LDS; then each wave walks members with lane (r, q) on
+// pixel (r, q) of the patch, adding its staged sum and its weight (recomputed from the group weight in
+// the filter's own arithmetic) to the tile in LDS.  The tile then adds to the accumulators once, as
 // the only writer of those pixels this pass (overflowing pairs are added by k_tile_overflow).
 // MIXED: the stage holds f16 samples, weighted and converted to fixed point here.
+//
+// The tile has a rim: a member's pixels outside the tile add to rim cells, which are never read, so a
+// pixel's cell is the member's cell plus the lane's and the walk has neither a bounds test nor a branch.
+// A list's last batch is filled up with members that add to spare columns.  Bound by VALU issue and the
+// 64-bit LDS adds.  3840x2160, 16 members, f16 stage, one / two channels, with positions, bounds and
+// 64-bit addresses worked out by every lane: 1005 / 336 us; this form
+// 816 / 333 us (reading the stage of the first, 2.8 GB with the tiles' overlap, takes 550 us).
 template <int C, bool MIXED, int KM>
 __global__ __launch_bounds__(256) void k_tile_gather(avd_collab_pass p, const uint32_t *__restrict__ members,
                                                      const float *__restrict__ group_weight, TileBins tiles,
@@ -2564,24 +2581,26 @@ __global__ __launch_bounds__(256) void k_tile_gather(avd_collab_pass p, const ui
                                                      int32_t *__restrict__ accum_second)
 {
     constexpr int T = 1 << kTileShift;
-    // Rows padded to 40 cells: the eight rows of a patch then fall on distinct banks (two passes
-    // per 64-bit add, the minimum, instead of eight).
-    constexpr int kRow = T + 8;
-    // Past the tile's cells, one trash cell per lane: a member pixel outside the tile adds there, so
-    // the walk has no branch (a branch let the compiler sink a member's staged load into it, where
-    // the lane then waited on it alone).  The trash is never read.
-    constexpr int kTrash = T * kRow;
-    __shared__ unsigned long long s_agg[T * kRow + 64];
-    __shared__ int32_t s_second[C == 2 ? T * kRow + 64 : 1];
-    __shared__ uint32_t s_id[256], s_pos[256];
-    __shared__ float s_sw[256];
+    // Seven cells of rim on every side; rows of 56 cells, so that four rows of 64-bit cells of a patch
+    // fall on distinct banks (two passes per add, the minimum) and eight of 32-bit ones do.
+    constexpr int kRim = 7, kRow = 56, kRows = T + 2 * kRim;
+    constexpr int kSpare = kRim * kRow + T + 2 * kRim + 1;  // a patch here ends in its row's last column
+    static_assert(kSpare % kRow + 8 <= kRow, "the spare columns hold a patch");
+    __shared__ unsigned long long s_agg[kRows * kRow];
+    __shared__ int32_t s_second[C == 2 ? kRows * kRow : 1];
+    struct __attribute__((aligned(16))) Entry {
+        uint32_t id;
+        int32_t cell;
+        float sw;
+    };
+    __shared__ Entry s_entry[256];
     const uint32_t tile = blockIdx.x;
     const uint32_t slot = tile / tiles.per_slot, in_slot = tile - slot * tiles.per_slot;
     const int ty = (int)(in_slot / tiles.tiles_x), tx = (int)(in_slot - ty * tiles.tiles_x);
     const int x0 = tx * T, y0 = ty * T;
     for (int i = threadIdx.x; i < T * kRow; i += 256) {
-        s_agg[i] = 0;
-        if (C == 2) s_second[i] = 0;
+        s_agg[kRim * kRow + i] = 0;
+        if (C == 2) s_second[kRim * kRow + i] = 0;
     }
     const uint32_t *list = tiles.list + (size_t)tile * tiles.cap;
     // The first entries are read with the count (a list always holds cap >= 256 entries, so the
@@ -2590,24 +2609,25 @@ __global__ __launch_bounds__(256) void k_tile_gather(avd_collab_pass p, const ui
     const uint32_t n = min(tiles.count[tile], tiles.cap);
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int r = lane >> 3, q = lane & 7;
+    const int lane_cell = r * kRow + q;
     const float kr_kq = p.kaiser[r] * p.kaiser[q];
     const float scale = p.accum_scale;
     const float kk_scale = kr_kq * scale;  // MIXED: the window and the fixed-point scale in one factor
     for (uint32_t base = 0; base < n; base += 256) {
         __syncthreads();
         const uint32_t k = base + threadIdx.x;
+        Entry mine{0u, kSpare, 0.0f};
         if (k < n) {
-            const uint32_t id = base == 0 ? id0 : list[k];
-            s_id[threadIdx.x] = id;
+            mine.id = base == 0 ? id0 : list[k];
             constexpr int KSHIFT = KM == 16 ? 4 : 3;
-            s_pos[threadIdx.x] = members[(size_t)(id >> KSHIFT) * (KM + 1) + (id & (KM - 1))];
-            s_sw[threadIdx.x] = group_weight[id >> KSHIFT] * p.weight_scale;
+            const uint32_t pos = members[(size_t)(mine.id >> KSHIFT) * (KM + 1) + (mine.id & (KM - 1))];
+            mine.cell = ((int)((pos >> 13) & 0x1FFF) - y0 + kRim) * kRow + (int)(pos & 0x1FFF) - x0 + kRim;
+            mine.sw = group_weight[mine.id >> KSHIFT] * p.weight_scale;
         }
+        s_entry[threadIdx.x] = mine;
         __syncthreads();
         const uint32_t batch = min(256u, n - base);
-        // kPer members per wave per step: every staged load is issued before the first add (the
-        // loads are unconditional, a lane past the batch reading the first member's row again, so
-        // none waits behind a branch).
+        // kPer members per wave per step: every staged load is issued before the first add.
         constexpr int kPer = 8;
         for (uint32_t e0 = wave; e0 < batch; e0 += 4 * kPer) {
             int32_t a[kPer], a2[kPer], wq[kPer];
@@ -2617,16 +2637,14 @@ __global__ __launch_bounds__(256) void k_tile_gather(avd_collab_pass p, const ui
             Staged v0[kPer], v1[kPer];
 #pragma unroll
             for (int u = 0; u < kPer; ++u) {
-                const uint32_t e = e0 + 4 * u;
-                const uint32_t ec = e < batch ? e : e0;
-                const uint32_t id = s_id[ec], pos = s_pos[ec];
-                sw[u] = s_sw[ec];
-                const int lx = (int)(pos & 0x1FFF) + q - x0, ly = (int)((pos >> 13) & 0x1FFF) + r - y0;
-                const bool in = e < batch && (unsigned)lx < (unsigned)T && (unsigned)ly < (unsigned)T;
-                cell[u] = in ? ly * kRow + lx : kTrash + lane;
-                const Staged *st = reinterpret_cast<const Staged *>(tiles.stage) + (size_t)id * C * 64 + lane;
-                v0[u] = st[0];
-                if (C == 2) v1[u] = st[64];
+                const Entry e = s_entry[e0 + 4 * u];
+                sw[u] = e.sw;
+                cell[u] = e.cell + lane_cell;
+                // The same member on every lane: a scalar base and the lane's own sample.
+                const Staged *st = reinterpret_cast<const Staged *>(tiles.stage) +
+                                   (size_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)e.id) * C * 64;
+                v0[u] = st[lane];
+                if (C == 2) v1[u] = st[64 + lane];
             }
 #pragma unroll
             for (int u = 0; u < kPer; ++u) {
@@ -2648,7 +2666,7 @@ __global__ __launch_bounds__(256) void k_tile_gather(avd_collab_pass p, const ui
                 } else {
                     a[u] = (int32_t)v0[u];
                     if (C == 2) a2[u] = (int32_t)v1[u];
-                    wq[u] = to_fixed_weight(sw[u] * kr_kq, scale);
+                    wq[u] = to_fixed_weight_up(sw[u] * kr_kq, scale);
                 }
             }
 #pragma unroll
@@ -2667,9 +2685,10 @@ __global__ __launch_bounds__(256) void k_tile_gather(avd_collab_pass p, const ui
         // The only writer of these pixels this pass: the adds need no result, so they are atomics
         // (the L2 does the read-modify-write and the workgroup does not wait for it).
         const size_t pix = (size_t)slot * px + (size_t)y * p.width + x;
-        const unsigned long long v = s_agg[ly * kRow + lx];
+        const int cell = (ly + kRim) * kRow + lx + kRim;
+        const unsigned long long v = s_agg[cell];
         if (v) atomicAdd(&aggregate[pix], v);
-        if (C == 2 && s_second[ly * kRow + lx]) atomicAdd(&accum_second[pix], s_second[ly * kRow + lx]);
+        if (C == 2 && s_second[cell]) atomicAdd(&accum_second[pix], s_second[cell]);
     }
 }
 
