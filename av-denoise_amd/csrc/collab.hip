@@ -1741,17 +1741,63 @@ __device__ __forceinline__ void dct8_inv(float *l)
     }
 }
 
+template <int CTRL>
+__device__ __forceinline__ float dpp_f32(float v)
+{
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xF, 0xF, true));
+}
+
+// Row (16 lanes) or half (32 lanes) swaps of four pairs: a keeps its even rows (its low half) and takes
+// b's, b keeps its odd rows (its high half) and takes a's.  In assembly, as the builtin's two results
+// come back as one register here; the wait states after the values' writes are the block's own.
+template <int XOR>
+__device__ __forceinline__ void swap_halves(float (&a)[4], float (&b)[4])
+{
+    if (XOR == 16)
+        asm("s_nop 1\n\tv_permlane16_swap_b32 %0, %4\n\tv_permlane16_swap_b32 %1, %5\n\t"
+            "v_permlane16_swap_b32 %2, %6\n\tv_permlane16_swap_b32 %3, %7\n\ts_nop 1"
+            : "+v"(a[0]), "+v"(a[1]), "+v"(a[2]), "+v"(a[3]), "+v"(b[0]), "+v"(b[1]), "+v"(b[2]), "+v"(b[3]));
+    else
+        asm("s_nop 1\n\tv_permlane32_swap_b32 %0, %4\n\tv_permlane32_swap_b32 %1, %5\n\t"
+            "v_permlane32_swap_b32 %2, %6\n\tv_permlane32_swap_b32 %3, %7\n\ts_nop 1"
+            : "+v"(a[0]), "+v"(a[1]), "+v"(a[2]), "+v"(a[3]), "+v"(b[0]), "+v"(b[1]), "+v"(b[2]), "+v"(b[3]));
+}
+
 // One Haar butterfly level between member lanes XOR (8, 16 or 32) apart.  `active` lanes take
-// part; a low lane keeps (low + high) * f, a high lane (low - high) * f, operands in the
-// reference's order.
+// part; a low lane keeps (low + high) * f, a high lane (low - high) * f.  Eight lanes apart the other
+// value is a rotation inside the DPP row, and a multiply-add by +-1 rounds as the sum or difference
+// does.  Further apart a permlane swap of two values brings both halves of one into the low lanes and of
+// the other into the high ones, and a second swap takes the results back.
 template <int XOR>
 __device__ __forceinline__ void haar_level(float (&v)[8], bool active, bool low)
 {
     const float f = 0.70710678118654752440f;
+    if (XOR == 8) {
+        const float sign = low ? 1.0f : -1.0f;
 #pragma unroll
-    for (int u = 0; u < 8; ++u) {
-        const float other = __shfl_xor(v[u], XOR);
-        if (active) v[u] = low ? (v[u] + other) * f : (other - v[u]) * f;
+        for (int u = 0; u < 8; ++u) {
+            const float t = __builtin_fmaf(v[u], sign, dpp_f32<0x128>(v[u])) * f;  // row_ror 8
+            v[u] = active ? t : v[u];
+        }
+        return;
+    }
+    float lo[4], hi[4], sum[4], diff[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        lo[i] = v[2 * i];
+        hi[i] = v[2 * i + 1];
+    }
+    swap_halves<XOR>(lo, hi);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        sum[i] = (lo[i] + hi[i]) * f;
+        diff[i] = (lo[i] - hi[i]) * f;
+    }
+    swap_halves<XOR>(sum, diff);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        v[2 * i] = active ? sum[i] : v[2 * i];
+        v[2 * i + 1] = active ? diff[i] : v[2 * i + 1];
     }
 }
 
@@ -1832,10 +1878,13 @@ __device__ __forceinline__ void group_inverse(float (&v)[HM][8], const HaarPlan 
     }
 }
 
+// Rounded half away from zero: the truncation plus the truncation of twice the rest, which is exact.
 __device__ __forceinline__ int32_t to_fixed(float v, float scale)
 {
-    const float c = fminf(fmaxf(v, -5.0f), 5.0f);
-    return (int32_t)roundf(c * scale);
+    const float c = fminf(fmaxf(v, -5.0f), 5.0f) * scale;
+    const int32_t i = (int32_t)c;
+    const float rest = c - (float)i;
+    return i + (int32_t)(rest + rest);
 }
 
 __device__ __forceinline__ int32_t to_fixed_weight(float w, float scale)
@@ -1863,6 +1912,9 @@ __device__ __forceinline__ void unpack_aggregate(unsigned long long v, int32_t &
 // `stage` ([ref][member][c][row][column] i32: a member's patch is 256 contiguous bytes per channel)
 // and the member enters the list of every 32x32 tile its patch overlaps; k_tile_gather then sums
 // them per tile.  KM group members: lane (m, q) holds column q of members m + 8 h, h < KM / 8.
+// Bound by VALU issue and, staged, by the stage's writes.  1920x1080 pooled, eight members, one / two
+// channels, alone: with the Haar levels through LDS permutes and the pooled threshold's nine divisions
+// and root in every lane 184 / 93 us; with swaps, DPP and those once per workgroup 170 / 85 us.
 template <int C, bool STAGED, int KM>
 __global__ __launch_bounds__(kWaves * 64) void k_collab_filter(avd_collab_pass p, const float *__restrict__ values,
                                                                const uint32_t *__restrict__ nslots,
@@ -1878,6 +1930,17 @@ __global__ __launch_bounds__(kWaves * 64) void k_collab_filter(avd_collab_pass p
     // threshold lambda sqrt(variance), the same f32 expressions for every reference, once per
     // workgroup.
     __shared__ float s_cvs[C][64], s_thr[C][64];
+    // The pooled threshold's divisions and roots, per column frequency u, and per channel and row
+    // frequency v, once per workgroup too.
+    __shared__ __align__(16) float s_inv_profile[8];
+    __shared__ float s_inv_row[C][8], s_own[C][8];
+    if (threadIdx.x < 8) s_inv_profile[threadIdx.x] = 1.0f / fmaxf(p.profile[threadIdx.x], 1e-20f);
+    if (threadIdx.x < 8 * C) {
+        const int c = threadIdx.x >> 3, v = threadIdx.x & 7;
+        const float lv = (p.sigma[c] * p.sigma[c]) * p.profile[v];
+        s_inv_row[c][v] = 1.0f / fmaxf(lv, 1e-20f);
+        s_own[c][v] = p.lambda[c] * sqrtf(lv * p.profile[0]);
+    }
     if (threadIdx.x < 64 * C) {
         const int c = threadIdx.x >> 6, v = (threadIdx.x >> 3) & 7, u = threadIdx.x & 7;
         const float cvs = (p.sigma[c] * p.sigma[c]) * (p.profile[u] * p.profile[v]);
@@ -1948,7 +2011,7 @@ __global__ __launch_bounds__(kWaves * 64) void k_collab_filter(avd_collab_pass p
             // then right) must reach threshold^2 times the in-range neighbour count; the spatial DC
             // takes its own test at lambda and the group DC is always kept.
             const float lv = sig2 * pv;
-            const float li = 1.0f / fmaxf(lv, 1e-20f);
+            const float li = s_inv_row[c][v], own_bar = s_own[c][v];
             const bool has_up = v > 0, has_down = v < 7;
             const float vertical = 1.0f + (has_up ? 1.0f : 0.0f) + (has_down ? 1.0f : 0.0f);
             const float threshold = lam * p.pool_ratio;
@@ -1962,19 +2025,20 @@ __global__ __launch_bounds__(kWaves * 64) void k_collab_filter(avd_collab_pass p
                 float e[8];
 #pragma unroll
                 for (int u = 0; u < 8; ++u)
-                    e[u] = row[h][u] * row[h][u] * li * (1.0f / fmaxf(p.profile[u], 1e-20f));
+                    e[u] = row[h][u] * row[h][u] * li * s_inv_profile[u];
                 if (v == 0) e[0] = 0.0f;
                 kept_profile[h] = 0.0f;
 #pragma unroll
                 for (int u = 0; u < 8; ++u) {
-                    const float above = __shfl_up(e[u], 1), below = __shfl_down(e[u], 1);
+                    // row_shr 1 and row_shl 1: a member's eight lanes lie in one DPP row.
+                    const float above = dpp_f32<0x111>(e[u]), below = dpp_f32<0x101>(e[u]);
                     float sum = e[u] + (has_down ? below : 0.0f) + (has_up ? above : 0.0f);
                     if (u > 0) sum += e[u - 1];
                     if (u < 7) sum += e[u + 1];
                     const float bar_u = u == 0 ? bar_first : (u == 1 ? bar_second : (u == 7 ? bar_last : bar_middle));
                     bool keep = sum >= bar_u;
                     if (u == 0) {
-                        const bool own = fabsf(row[h][0]) >= lam * sqrtf(lv * p.profile[0]);
+                        const bool own = fabsf(row[h][0]) >= own_bar;
                         if (v == 0) keep = own;
                         if (m == 0 && h == 0) keep = keep || v == 0;
                     }
@@ -2021,9 +2085,9 @@ __global__ __launch_bounds__(kWaves * 64) void k_collab_filter(avd_collab_pass p
             }
         }
         float sum = part;
-        sum += __shfl_xor(sum, 1);
-        sum += __shfl_xor(sum, 2);
-        sum += __shfl_xor(sum, 4);
+        sum += dpp_f32<0xB1>(sum);   // quad_perm 1,0,3,2
+        sum += dpp_f32<0x4E>(sum);   // quad_perm 2,3,0,1
+        sum += dpp_f32<0x141>(sum);  // row_half_mirror: the other quad, whose lanes agree
         const float weight = (isnan(sum) || isinf(sum)) ? 0.0f : 1.0f / fmaxf(sum, 1e-12f);
         if (c == 0) {
             if (live && lane == 0) group_weight[ref] = weight;
