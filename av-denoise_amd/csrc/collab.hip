@@ -848,8 +848,9 @@ constexpr int kPrepRows = 8, kPrepCols = 248;
 template <int C>
 __global__ __launch_bounds__(256) void k_centre_prep(const uint16_t *__restrict__ frame, int W, int H,
                                                      uint16_t *__restrict__ plane, uint16_t *__restrict__ plane_odd,
-                                                     uint32_t *__restrict__ energy)
+                                                     uint32_t *__restrict__ energy, uint32_t *__restrict__ redo_count)
 {
+    if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) *redo_count = 0;  // the search adds to it
     constexpr int kRead = kPrepRows + 7, kRun = 8, kRuns = kPrepCols / kRun;
     __shared__ __align__(16) uint32_t s_col[kPrepRows][kPrepCols + 8];
     const int t = threadIdx.x, x0 = blockIdx.x * kPrepCols, y0 = blockIdx.y * kPrepRows;
@@ -2923,16 +2924,15 @@ hipError_t launch_centre_km(const avd_collab_pass &p, const uint16_t *codes, uin
         const dim3 pg(div_up(W, kPrepCols), div_up(H, kPrepRows));
         const int refs_x = (W - 8 + st - 1) / st + 1, refs_y = (H - 8 + st - 1) / st + 1;
         const unsigned gm = div_up(((refs_x + 1) / 2) * ((refs_y + 3) / 4), kWaves);
-        const hipError_t e = launch_fill_u32(centre->redo, 0, 1, s);
-        if (e != hipSuccess) return e;
         if (p.channels == 1) {
-            k_centre_prep<1><<<pg, 256, 0, s>>>(frame, W, H, centre->plane, centre->plane_odd, centre->energy);
+            k_centre_prep<1><<<pg, 256, 0, s>>>(frame, W, H, centre->plane, centre->plane_odd, centre->energy,
+                                              centre->redo);
             k_centre_mfma<1, KM><<<gm, blk, 0, s>>>(p, codes, centre->plane,
                                                     (uint32_t)(centre->plane_odd - centre->plane), centre->energy,
                                                     members, centre->redo, nullptr);
             k_centre_redo<1, KM><<<kRedoBlocks, blk, 0, s>>>(p, codes, centre->redo, members);
         } else {
-            k_centre_prep<2><<<pg, 256, 0, s>>>(frame, W, H, centre->plane, nullptr, centre->energy);
+            k_centre_prep<2><<<pg, 256, 0, s>>>(frame, W, H, centre->plane, nullptr, centre->energy, centre->redo);
             k_centre_mfma<2, KM><<<gm, blk, 0, s>>>(p, codes, centre->plane, 0u, centre->energy, members,
                                                     centre->redo, nullptr);
             k_centre_redo<2, KM><<<kRedoBlocks, blk, 0, s>>>(p, codes, centre->redo, members);
@@ -3130,15 +3130,15 @@ hipError_t launch_collab_filter_binned(const avd_collab_pass &p, const float *va
 {
     if (mixed && p.pool_ratio > 0.0f) return hipErrorInvalidValue;  // the mixed form thresholds hard
     if (!pass_ok(p) || (p.channels == 2 && !accum_second) || !tiles.stage || !tiles.count || !tiles.list ||
-        !tiles.overflow || !tiles.overflow_count || tiles.cap < kTileCapMin ||
+        !tiles.overflow || tiles.cap < kTileCapMin ||
         tiles.tiles_x != (p.width + (1u << kTileShift) - 1) >> kTileShift ||
         tiles.per_slot != tiles.tiles_x * ((p.height + (1u << kTileShift) - 1) >> kTileShift))
         return hipErrorInvalidValue;
     hipError_t e = upload_taps(s);
     if (e != hipSuccess) return e;
     const uint32_t n_tiles = tiles.per_slot * p.slots;
-    e = launch_fill_u32(tiles.count, 0, n_tiles, s);
-    if (e == hipSuccess) e = launch_fill_u32(tiles.overflow_count, 0, 1, s);
+    if (tiles.overflow_count != tiles.count + n_tiles) return hipErrorInvalidValue;
+    e = launch_fill_u32(tiles.count, 0, n_tiles + 1, s);  // the overflow count ends the tiles' counts
     if (e != hipSuccess) return e;
     const uint32_t refs = (uint32_t)ref_count(p);
     if (p.group_size == 16) {

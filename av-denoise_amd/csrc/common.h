@@ -185,7 +185,7 @@ inline uint32_t tile_cap_for(uint32_t group_size) { return group_size == 16 ? 20
 constexpr uint32_t kTileCapMin = 256;  // the gather reads a list's first 256 entries with its count
 struct TileBins {
     int32_t *stage;
-    uint32_t *count, *list, *overflow, *overflow_count;
+    uint32_t *count, *list, *overflow, *overflow_count;  // overflow_count follows the last tile's count
     uint32_t tiles_x, per_slot;  // tiles per row, tiles per ring slot
     uint32_t cap;                // entries per tile list (at least kTileCapMin)
 };
