@@ -2907,8 +2907,8 @@ bool centre_on_matrix_cores(const avd_collab_pass &p)
 
 namespace {
 
-// Workgroups of the exact centre search over the redo list (a grid-stride loop over the list's
-// count; a few percent of a 4K frame's references when a lane's short list runs out).
+// Workgroups of the exact centre search over the redo list (a grid-stride loop over the list's count):
+// full-range noise can put every reference there, ordinary content a few.
 constexpr unsigned kRedoBlocks = 1024;
 
 template <int KM>
