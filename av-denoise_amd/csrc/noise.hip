@@ -278,7 +278,8 @@ __device__ __forceinline__ float fold8(const float (&v)[8])
 }
 __device__ __forceinline__ float fold4(const float (&v)[4]) { return (v[0] + v[2]) + (v[1] + v[3]); }
 
-// fminf / fmaxf without the quieting multiply a load would get first.
+// fminf / fmaxf without the quieting operation a load would get first: their operands hold no signalling
+// NaN (which this instruction passes on, where it drops a quiet one).
 __device__ __forceinline__ float min_f(float a, float b)
 {
     float r;
@@ -377,7 +378,8 @@ __global__ __launch_bounds__(kTThreads) void k_temporal_stats(const float *__res
 #pragma unroll
         for (int r = 0; r < kTB; ++r) {
             const bool in = in_x && r < k.bh;
-            s_new[dst + r * kTB] = in ? a[r] : 0.0f;
+            // Quiet, for the extremes: every other use only adds.
+            s_new[dst + r * kTB] = in ? __builtin_canonicalizef(a[r]) : 0.0f;
             if constexpr (COMP) {
                 s_old[dst + r * kTB] = in ? b[r] : 0.0f;
                 // A pixel whose match leaves the frame takes no part: its residual along the vector is
@@ -586,8 +588,10 @@ __global__ __launch_bounds__(kTThreads) void k_temporal_stats(const float *__res
     }
     if (role != 3) return;
     // The quarter's luma, sum_d and sum_d2 trees and its extremes over the pixels in the frame, four
-    // columns at a time (columns c and c + 4 are the tree's first pairs).
-    float luma[4], sum_d[4], sum_d2[4], lo = 1.0e30f, hi = -1.0e30f;
+    // columns at a time (columns c and c + 4 are the tree's first pairs).  The extremes start from NaN,
+    // which any value replaces, so that a quarter of values past +-1e30 keeps its own and one of NaNs alone
+    // is NaN; a pixel past the frame is +-1e30.
+    float luma[4], sum_d[4], sum_d2[4], lo = __builtin_nanf(""), hi = lo;
 #pragma unroll 1
     for (int half = 0; half < 2; ++half) {
         float n[4][8], d[4][8], d2[4][8];
