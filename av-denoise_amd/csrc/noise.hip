@@ -12,6 +12,7 @@
 // turn; each total then adds its 256 thread sums in thread order, as does each tile in stage 1),
 // so the totals are bit-identical to the reference's.  The work is one read of the frame (HBM).
 
+#include <algorithm>
 #include <mutex>
 #include <type_traits>
 
@@ -37,6 +38,9 @@ constexpr int kReduceBlock = 256;               // stage 2's threads (noise/mod.
 // order.  Bound by that chain and the loads it waits for, hidden by the eight workgroups a CU holds.
 // 3840x2160 luma: 18.6 us with a thread per pixel and eight tiles' chains per workgroup, 9.8 us now.
 constexpr int kTileRows = 2, kPlanes = 16;
+// Workgroups along y of a grid layer; a taller frame (past 2^19 rows) takes further layers along z, as a
+// grid's y extent is limited to 16 bits.
+constexpr uint32_t kGridRows = 1u << 15;
 constexpr int kPlaneStride = kImmBlockX * kImmBlockY + 32;
 
 // Where columns 4 g .. 4 g + 3 of row 0 of LDS plane i start: neighbouring planes 32 banks apart and the
@@ -52,7 +56,9 @@ __global__ __launch_bounds__(256) void k_noise_partial(const float *__restrict__
     __shared__ __align__(16) float s_abs[kPlanes * kPlaneStride];
     const int t = (int)threadIdx.x, c = t % C, col = t / C;
     const int tiles_x = (W + kImmBlockX - 1) / kImmBlockX, tiles_y = (H + kImmBlockY - 1) / kImmBlockY;
-    const int x = (int)blockIdx.x * kCols + col, y0 = (int)blockIdx.y * kRows;
+    const int group_y = (int)(blockIdx.z * kGridRows + blockIdx.y);
+    if (group_y > (H - 1) / kRows) return;  // the last layer's surplus: whole workgroups
+    const int x = (int)blockIdx.x * kCols + col, y0 = group_y * kRows;
     const size_t pitch = (size_t)W * C;
     const float *f = ring + (size_t)frame * W * H * C + c;
     const bool in_x = x >= 1 && x < W - 1;
@@ -90,7 +96,7 @@ __global__ __launch_bounds__(256) void k_noise_partial(const float *__restrict__
 #pragma unroll
         for (int g = 0; g < kImmBlockX / 4; ++g) sum = (((sum + v[g].x) + v[g].y) + v[g].z) + v[g].w;
     }
-    const int tx = (int)blockIdx.x * kTilesX + lane / C % kTilesX, ty = (int)blockIdx.y * kTileRows + lane / C / kTilesX;
+    const int tx = (int)blockIdx.x * kTilesX + lane / C % kTilesX, ty = group_y * kTileRows + lane / C / kTilesX;
     if (tx < tiles_x && ty < tiles_y) {
         float *out = partials + ((size_t)ty * tiles_x + tx) * kImmLanes;
         out[lane % C] = sum;
@@ -171,7 +177,8 @@ hipError_t launch_noise_spatial(const float *ring, uint32_t width, uint32_t heig
         (uint64_t)width * height * channels * (frame + 1ull) > (1ull << 40))
         return hipErrorInvalidValue;
     const uint32_t tiles_x = (width + kImmBlockX - 1) / kImmBlockX, tiles_y = (height + kImmBlockY - 1) / kImmBlockY;
-    const dim3 grid(div_up(width, 256 / channels), div_up(height, kTileRows * kImmBlockY));
+    const uint32_t rows = div_up(height, kTileRows * kImmBlockY);
+    const dim3 grid(div_up(width, 256 / channels), std::min(rows, kGridRows), div_up(rows, kGridRows));
     if (channels == 1)
         k_noise_partial<1><<<grid, 256, 0, s>>>(ring, partials, frame, (int)width, (int)height);
     else
