@@ -222,6 +222,10 @@ SIGNATURES = {
     "avd_site_nlm_single": (ctypes.c_int, [ctypes.POINTER(NlmWindow), P, P, P, P, P, P]),
     "avd_site_nlm_pair": (ctypes.c_int, [ctypes.POINTER(NlmWindow), P, P, P, P, P, P, P, P, P]),
     "avd_site_nlm_finish": (ctypes.c_int, [P, P, P, P, f32, u32, u32, P, P]),
+    "avd_nlm_frame_for_test": (ctypes.c_int, [ctypes.POINTER(NlmWindow), u32, u32, u32, P, ctypes.POINTER(P),
+                                              ctypes.POINTER(P), ctypes.POINTER(P), ctypes.POINTER(P), P, f32, P, P, P,
+                                              P, P]),
+    "avd_tuning_sample_for_test": (f32, [u32, ctypes.c_uint64, u32, f32, f32]),
     "avd_site_noise_spatial": (ctypes.c_int, [P, u32, u32, u32, u32, P, P, u32, P]),
     "avd_site_noise_temporal_stats": (ctypes.c_int, [P, u32, u32, u32, u32, u32, P, u32, u32, u32, u32, u32, P, P]),
     "avd_site_noise_temporal_zero": (ctypes.c_int, [P, u32, P]),

@@ -675,4 +675,46 @@ avd_status avd_site_nlm_finish(const float *frame, const float *accum, const flo
                       "nlm_finish");
 }
 
+avd_status avd_nlm_frame_for_test(const avd_nlm_window *w, uint32_t form, uint32_t candidate, uint32_t pairs,
+                                  const float *centre, const float *const *fwd, const float *const *bwd,
+                                  const float *const *conf_fwd, const float *const *conf_bwd, const float *lut,
+                                  float self_weight, float *accum, float *wsum, float *maxw, float *out, void *stream)
+{
+    if (!w || !centre || (pairs && (!fwd || !bwd)) || !conf_fwd != !conf_bwd || !lut || !out ||
+        (form == AVD_NLM_FORM_PLAIN && (!accum || !wsum || !maxw)))
+        return fail(AVD_ERR_NULL_ARGUMENT, "null argument");
+    if (form > AVD_NLM_FORM_BATCHED || pairs > (uint32_t)avd::kNlmMaxPairs)
+        return fail(AVD_ERR_INVALID_OPTIONS, "unknown form or too many pairs");
+    const avd::NlmWindow k{(int)w->width, (int)w->height, (int)w->channels, (int)w->patch_radius, (int)w->search_radius,
+                           w->h2_inv_norm * 1.4426950408889634f, w->noise_offset, (int)w->step, (int)w->blocks_x,
+                           (int)w->blocks_y};
+    avd::NlmFrames f{};
+    f.pairs = (int)pairs;
+    for (uint32_t i = 0; i < pairs; ++i) {
+        f.fwd[i] = fwd[i];
+        f.bwd[i] = bwd[i];
+        f.conf_f[i] = conf_fwd ? conf_fwd[i] : nullptr;
+        f.conf_b[i] = conf_bwd ? conf_bwd[i] : nullptr;
+    }
+    const hipStream_t s = static_cast<hipStream_t>(stream);
+    if (form == AVD_NLM_FORM_BATCHED)
+        return hip_status(avd::launch_nlm_window(k, f, centre, lut, self_weight, out, s, (int)candidate), "nlm frame");
+    hipError_t e = hipSuccess;
+    for (uint32_t i = 0; i < pairs && e == hipSuccess; ++i)
+        e = avd::launch_nlm_pair(k, centre, f.fwd[i], f.bwd[i], f.conf_f[i], f.conf_b[i], accum, wsum, maxw, s,
+                                 (int)candidate, i == 0);
+    if (e == hipSuccess)
+        e = avd::launch_nlm_single(k, centre, lut, accum, wsum, maxw, s, (int)candidate, pairs == 0, self_weight, out);
+    return hip_status(e, "nlm frame");
+}
+
+float avd_tuning_sample_for_test(uint32_t confidence, uint64_t index, uint32_t patch_radius, float h2_inv_norm,
+                                 float noise_offset)
+{
+    if (confidence)
+        return avd::kTuneConfidenceLow + avd::kTuneConfidenceSpan * avd::hashed_unit(index, avd::kTuneConfidence);
+    const float spread = avd::tuning_spread((int)patch_radius, h2_inv_norm, noise_offset);
+    return 0.5f - 0.5f * spread + spread * avd::hashed_unit(index, avd::kTuneFrames);
+}
+
 }  // extern "C"

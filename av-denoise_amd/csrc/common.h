@@ -20,6 +20,16 @@ hipError_t launch_egress(const float *frame, uint32_t *p0, uint32_t *p1, uint32_
                          int samples_per_word, float max_value, hipStream_t s);
 hipError_t launch_copy_words(const uint32_t *src, uint32_t *dst, uint64_t words, hipStream_t s);
 hipError_t launch_fill_u32(void *dst, uint32_t value, uint64_t words, hipStream_t s);
+// Sample i of stream `seed`: a fixed hash of both, uniform in [0, 1).
+__host__ __device__ inline float hashed_unit(uint64_t i, uint32_t seed)
+{
+    uint32_t h = (uint32_t)i * 0x9E3779B1u + (uint32_t)(i >> 32) * 0x85EBCA77u + seed * 0xC2B2AE3Du;
+    h = (h ^ h >> 16) * 0x7FEB352Du;
+    h = (h ^ h >> 15) * 0x846CA68Bu;
+    return (float)((h ^ h >> 16) >> 8) * (1.0f / 16777216.0f);
+}
+// dst[i] = low + span * hashed_unit(i, seed).
+hipError_t launch_fill_samples(float *dst, uint64_t n, uint32_t seed, float low, float span, hipStream_t s);
 
 // ---- nlm.hip ----------------------------------------------------------------------------
 struct NlmWindow {

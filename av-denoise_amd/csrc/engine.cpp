@@ -557,65 +557,75 @@ NlmWindow NlmPass::window() const
     return w;
 }
 
-// The window launch sites' rows per wave, picked by the tuner on this pass's own buffers: ring
-// slots of flat mid-grey (the window walks every offset whatever the content, so the time is the
-// content's) and, with confidence, blocks of confidence 1.  The stream then starts from scratch.
+// The window launch sites' columns per lane, picked by the tuner on this pass's own buffers: ring slots,
+// confidences and sums of hashed samples (see tuning_spread; the window walks every offset whatever the
+// content, so the time is the content's).  The stream then starts from scratch.
 void NlmPass::tune_windows()
 {
     const size_t px = (size_t)W_ * H_;
-    check_hip(launch_fill_u32(ring_.values.ptr, 0x3f000000u, px * C_ * ring_.N, stream_), "tuning frames");
+    const float spread = tuning_spread((int)P_, h2_, offset_);
+    check_hip(launch_fill_samples(ring_.values.as<float>(), px * C_ * ring_.N, kTuneFrames, 0.5f - 0.5f * spread,
+                                  spread, stream_),
+              "tuning frames");
+    const size_t blocks = (size_t)mg_.blocks_x * mg_.blocks_y;
     if (confidence_)
-        check_hip(launch_fill_u32(conf_.ptr, 0x3f800000u, conf_.bytes / sizeof(float), stream_), "tuning confidence");
+        check_hip(launch_fill_samples(conf_.as<float>(), 2 * r_ * blocks, kTuneConfidence, kTuneConfidenceLow,
+                                      kTuneConfidenceSpan, stream_),
+                  "tuning confidence");
     const NlmWindow w = window();
-    auto clear = [&]() -> hipError_t {
-        hipError_t e = launch_fill_u32(accum_.ptr, 0, px * C_, stream_);
-        if (e == hipSuccess) e = launch_fill_u32(wsum_.ptr, 0, px, stream_);
-        if (e == hipSuccess) e = launch_fill_u32(maxw_.ptr, 0, px, stream_);
+    float *const accum = accum_.as<float>(), *const wsum = wsum_.as<float>(), *const maxw = maxw_.as<float>();
+    float *const out = outputs_[0].as<float>();
+    auto clear_sums = [&]() -> hipError_t {
+        hipError_t e = launch_fill_samples(accum, px * C_, kTuneSums, 0.0f, 8.0f, stream_);
+        if (e == hipSuccess) e = launch_fill_samples(wsum, px, kTuneSums, 1.0f, 8.0f, stream_);
+        if (e == hipSuccess) e = launch_fill_samples(maxw, px, kTuneSums, 0.0f, 1.0f, stream_);
         return e;
     };
-    auto read = [&]() {
-        std::vector<uint8_t> out(px * (C_ + 2) * sizeof(float));
-        check_hip(hipMemcpy(out.data(), accum_.ptr, px * C_ * sizeof(float), hipMemcpyDeviceToHost), "tuning read");
-        check_hip(hipMemcpy(out.data() + px * C_ * 4, wsum_.ptr, px * sizeof(float), hipMemcpyDeviceToHost),
-                  "tuning read");
-        check_hip(hipMemcpy(out.data() + px * (C_ + 1) * 4, maxw_.ptr, px * sizeof(float), hipMemcpyDeviceToHost),
-                  "tuning read");
-        return out;
+    auto clear_frame = [&]() -> hipError_t { return launch_fill_u32(out, 0, px * C_, stream_); };
+    auto read_into = [&](std::vector<uint8_t> &to, const float *from, size_t n) {
+        const size_t at = to.size();
+        to.resize(at + n * sizeof(float));
+        check_hip(hipMemcpy(to.data() + at, from, n * sizeof(float), hipMemcpyDeviceToHost), "tuning read");
+    };
+    auto read_sums = [&]() {
+        std::vector<uint8_t> o;
+        read_into(o, accum, px * C_);
+        read_into(o, wsum, px);
+        read_into(o, maxw, px);
+        return o;
+    };
+    auto read_frame = [&]() {
+        std::vector<uint8_t> o;
+        read_into(o, out, px * C_);
+        return o;
     };
     const std::string key = "C" + std::to_string(C_) + " P" + std::to_string(P_) + " S" + std::to_string(S_) + " " +
                             std::to_string(W_) + "x" + std::to_string(H_);
     const float *f = ring_.value_slot(0);
     variant_single_ = Tuner::instance().choose(
         "nlm_single", key, kNlmVariants, stream_,
-        [&](int v) { return launch_nlm_single(w, f, lut_.as<float>(), accum_.as<float>(), wsum_.as<float>(),
-                                              maxw_.as<float>(), stream_, v); },
-        clear, read);
-    {
-        NlmFrames fr{};
-        fr.pairs = (int)r_;
-        for (uint32_t k = 0; k < r_; ++k) {
-            fr.fwd[k] = fr.bwd[k] = f;
-            fr.conf_f[k] = fr.conf_b[k] = confidence_ ? conf_.as<float>() : nullptr;
-        }
-        float *out = outputs_[0].as<float>();
-        variant_window_ = Tuner::instance().choose(
-            "nlm_window", key + " r" + std::to_string(r_) + (confidence_ ? " confidence" : ""), kNlmBatchedVariants,
-            stream_, [&](int v) { return launch_nlm_window(w, fr, f, lut_.as<float>(), self_weight_, out, stream_, v); },
-            [&]() -> hipError_t { return launch_fill_u32(out, 0, px * C_, stream_); },
-            [&]() {
-                std::vector<uint8_t> o(px * C_ * sizeof(float));
-                check_hip(hipMemcpy(o.data(), out, o.size(), hipMemcpyDeviceToHost), "tuning read");
-                return o;
-            });
+        [&](int v) { return launch_nlm_single(w, f, lut_.as<float>(), accum, wsum, maxw, stream_, v); }, clear_sums,
+        read_sums);
+    NlmFrames fr{};
+    fr.pairs = (int)r_;
+    for (uint32_t k = 0; k < r_; ++k) {
+        fr.fwd[k] = ring_.value_slot(1 + 2 * k);
+        fr.bwd[k] = ring_.value_slot(2 + 2 * k);
+        fr.conf_f[k] = confidence_ ? conf_.as<float>() + 2 * k * blocks : nullptr;
+        fr.conf_b[k] = confidence_ ? conf_.as<float>() + (2 * k + 1) * blocks : nullptr;
     }
-    if (r_ > 0) {
-        const float *c = confidence_ ? conf_.as<float>() : nullptr;
+    variant_window_ = Tuner::instance().choose(
+        "nlm_window", key + " r" + std::to_string(r_) + (confidence_ ? " confidence" : ""), kNlmBatchedVariants,
+        stream_, [&](int v) { return launch_nlm_window(w, fr, f, lut_.as<float>(), self_weight_, out, stream_, v); },
+        clear_frame, read_frame);
+    if (r_ > 0)
         variant_pair_ = Tuner::instance().choose(
-            "nlm_pair", key + (c ? " confidence" : ""), kNlmVariants, stream_,
-            [&](int v) { return launch_nlm_pair(w, f, f, f, c, c, accum_.as<float>(), wsum_.as<float>(),
-                                                maxw_.as<float>(), stream_, v); },
-            clear, read);
-    }
+            "nlm_pair", key + (confidence_ ? " confidence" : ""), kNlmVariants, stream_,
+            [&](int v) {
+                return launch_nlm_pair(w, f, fr.fwd[0], fr.bwd[0], fr.conf_f[0], fr.conf_b[0], accum, wsum, maxw,
+                                       stream_, v);
+            },
+            clear_sums, read_sums);
 }
 
 size_t NlmPass::max_held() const { return r_; }

@@ -242,7 +242,7 @@ class NlmPass : public Pass {
     DeviceBuffer outputs_[2];
     bool ready_ = false;
     int ready_output_ = 0, next_output_ = 0;
-    int variant_single_ = 0, variant_pair_ = 0;  // the tuner's rows per wave of the window sites
+    int variant_single_ = 0, variant_pair_ = 0;  // the tuner's columns per lane of the window sites
     int variant_window_ = 0;                     // and of the batched form's window
     bool batched_ = false;                       // every window of a frame in one launch
     uint32_t tail_remaining_ = 0;

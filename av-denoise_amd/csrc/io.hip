@@ -79,6 +79,13 @@ __global__ __launch_bounds__(kThreads) void k_fill_u32(uint32_t *__restrict__ ds
         dst[i] = value;
 }
 
+__global__ __launch_bounds__(kThreads) void k_fill_samples(float *__restrict__ dst, uint64_t n, uint32_t seed, float low,
+                                                          float span)
+{
+    for (uint64_t i = (uint64_t)blockIdx.x * kThreads + threadIdx.x; i < n; i += (uint64_t)gridDim.x * kThreads)
+        dst[i] = low + span * hashed_unit(i, seed);
+}
+
 // A grid-stride launch sized to keep every CU busy without an oversized grid.
 inline unsigned grid_for(uint64_t items)
 {
@@ -118,6 +125,13 @@ hipError_t launch_copy_words(const uint32_t *src, uint32_t *dst, uint64_t words,
 {
     if (words == 0) return hipSuccess;
     k_copy_words<<<grid_for(words), kThreads, 0, s>>>(src, dst, words);
+    return hipGetLastError();
+}
+
+hipError_t launch_fill_samples(float *dst, uint64_t n, uint32_t seed, float low, float span, hipStream_t s)
+{
+    if (n == 0) return hipSuccess;
+    k_fill_samples<<<grid_for(n), kThreads, 0, s>>>(dst, n, seed, low, span);
     return hipGetLastError();
 }
 

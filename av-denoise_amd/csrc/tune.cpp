@@ -1,6 +1,7 @@
 #include "tune.h"
 
 #include <algorithm>
+#include <cmath>
 #include <mutex>
 
 #include "engine.h"
@@ -16,6 +17,13 @@ std::vector<TuneEntry> g_entries;
 constexpr int kReps = 3;
 
 }  // namespace
+
+float tuning_spread(int patch_radius, float h2_inv_norm, float offset)
+{
+    // The mean squared difference of two uniform samples is spread^2 / 6; a patch sums 3 of it per pixel.
+    const float side = 2.0f * (float)patch_radius + 1.0f;
+    return std::min(std::sqrt(2.0f * (1.0f / h2_inv_norm + offset)) / side, 1.0f);
+}
 
 Tuner &Tuner::instance()
 {

@@ -19,6 +19,14 @@ struct TuneEntry {
     std::vector<double> ms;  // best time of each candidate (negative: did not match the baseline)
 };
 
+// The content the NLM window sites are tuned on: samples 0.5 + spread (u - 0.5), u uniform, with the spread
+// at which two random patches lie one weight scale (1 / h2) past the noise offset, so that weights vary with
+// every sample and with every index a launch could get wrong (flat content gives every offset one weight and
+// any two launches the same sums).  Confidences lie in [0.25, 1).
+constexpr uint32_t kTuneFrames = 1, kTuneConfidence = 2, kTuneSums = 3;  // streams of hashed_unit
+constexpr float kTuneConfidenceLow = 0.25f, kTuneConfidenceSpan = 0.75f;
+float tuning_spread(int patch_radius, float h2_inv_norm, float offset);
+
 class Tuner {
   public:
     static Tuner &instance();

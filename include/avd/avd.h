@@ -312,7 +312,7 @@ avd_status avd_host_denoiser_window_span(const avd_host_denoiser *denoiser, avd_
 
 /* ---- launch-site tuner (KernelSelector, tune/selector.rs:109; VariantSite, tune/site.rs:56-157) -- */
 
-/* An engine's tunable launch sites (the NLM windows' rows per wave; the NL4D trajectory search's
+/* An engine's tunable launch sites (the NLM windows' columns per lane; the NL4D trajectory search's
  * references per wave) offer candidate launches that compute bit-identical outputs.  With tuning on
  * (the default) the first engine of a shape runs every candidate on its own buffers, drops any whose
  * outputs differ from the baseline's (candidate 0) by a bit, times the rest with HIP events and
@@ -440,6 +440,20 @@ avd_status avd_site_nlm_pair(const avd_nlm_window *w, const float *centre, const
                              void *stream);
 avd_status avd_site_nlm_finish(const float *frame, const float *accum, const float *wsum, const float *maxw,
                                float self_weight, uint32_t pixels, uint32_t channels, float *out, void *stream);
+
+/* One frame's windows and finish as an engine launches them in `form` (plain or batched) by the tuner's
+ * candidate `candidate` of every launch: `pairs` pairs, oldest first (`fwd[k]` and `bwd[k]` device frames,
+ * `conf_fwd[k]` and `conf_bwd[k]` their confidences, or both arrays null), then the single window, which
+ * finishes into `out`.  accum, wsum and maxw are the plain form's sums and need no clearing.  For tests of the
+ * candidates, whose outputs are bit-identical. */
+avd_status avd_nlm_frame_for_test(const avd_nlm_window *w, uint32_t form, uint32_t candidate, uint32_t pairs,
+                                  const float *centre, const float *const *fwd, const float *const *bwd,
+                                  const float *const *conf_fwd, const float *const *conf_bwd, const float *lut,
+                                  float self_weight, float *accum, float *wsum, float *maxw, float *out, void *stream);
+/* Sample `index` of the frames (`confidence` 0) or confidences the tuner fills its buffers with for windows of
+ * this patch radius, weight scale and noise offset.  For tests of what its comparison of candidates can see. */
+float avd_tuning_sample_for_test(uint32_t confidence, uint64_t index, uint32_t patch_radius, float h2_inv_norm,
+                                 float noise_offset);
 
 /* Spatial noise measurement: both stages of the Immerkaer estimate of frame `frame` of a ring of
  * f32 [frame][height][width][channels] samples (run_noise_estimate, noise/spatial.rs:93-125, with
