@@ -557,9 +557,9 @@ NlmWindow NlmPass::window() const
     return w;
 }
 
-// The window launch sites' columns per lane, picked by the tuner on this pass's own buffers: ring slots,
-// confidences and sums of hashed samples (see tuning_spread; the window walks every offset whatever the
-// content, so the time is the content's).  The stream then starts from scratch.
+// The window launch sites' columns per lane, picked by the tuner on this pass's own buffers, each launch as
+// denoise() makes it: ring slots, confidences and sums of hashed samples (see tuning_spread; the window walks
+// every offset whatever the content, so the time is the content's).  The stream then starts from scratch.
 void NlmPass::tune_windows()
 {
     const size_t px = (size_t)W_ * H_;
@@ -581,7 +581,10 @@ void NlmPass::tune_windows()
         if (e == hipSuccess) e = launch_fill_samples(maxw, px, kTuneSums, 0.0f, 1.0f, stream_);
         return e;
     };
-    auto clear_frame = [&]() -> hipError_t { return launch_fill_u32(out, 0, px * C_, stream_); };
+    auto clear_frame = [&]() -> hipError_t {
+        const hipError_t e = clear_sums();
+        return e == hipSuccess ? launch_fill_u32(out, 0, px * C_, stream_) : e;
+    };
     auto read_into = [&](std::vector<uint8_t> &to, const float *from, size_t n) {
         const size_t at = to.size();
         to.resize(at + n * sizeof(float));
@@ -603,9 +606,11 @@ void NlmPass::tune_windows()
                             std::to_string(W_) + "x" + std::to_string(H_);
     const float *f = ring_.value_slot(0);
     variant_single_ = Tuner::instance().choose(
-        "nlm_single", key, kNlmVariants, stream_,
-        [&](int v) { return launch_nlm_single(w, f, lut_.as<float>(), accum, wsum, maxw, stream_, v); }, clear_sums,
-        read_sums);
+        "nlm_single", key + (r_ == 0 ? " alone" : ""), kNlmVariants, stream_,
+        [&](int v) {
+            return launch_nlm_single(w, f, lut_.as<float>(), accum, wsum, maxw, stream_, v, r_ == 0, self_weight_, out);
+        },
+        clear_frame, read_frame);
     NlmFrames fr{};
     fr.pairs = (int)r_;
     for (uint32_t k = 0; k < r_; ++k) {
@@ -618,12 +623,12 @@ void NlmPass::tune_windows()
         "nlm_window", key + " r" + std::to_string(r_) + (confidence_ ? " confidence" : ""), kNlmBatchedVariants,
         stream_, [&](int v) { return launch_nlm_window(w, fr, f, lut_.as<float>(), self_weight_, out, stream_, v); },
         clear_frame, read_frame);
-    if (r_ > 0)
+    if (r_ > 0)  // one pair a frame starts the sums, more add to them
         variant_pair_ = Tuner::instance().choose(
-            "nlm_pair", key + (confidence_ ? " confidence" : ""), kNlmVariants, stream_,
+            "nlm_pair", key + (confidence_ ? " confidence" : "") + (r_ == 1 ? " alone" : ""), kNlmVariants, stream_,
             [&](int v) {
                 return launch_nlm_pair(w, f, fr.fwd[0], fr.bwd[0], fr.conf_f[0], fr.conf_b[0], accum, wsum, maxw,
-                                       stream_, v);
+                                       stream_, v, r_ == 1);
             },
             clear_sums, read_sums);
 }

@@ -81,3 +81,19 @@ def test_the_tuner_drops_none(chroma, W, H, P, S, r, hq):
     assert {e["site"] for e in entries} == {"nlm_single", "nlm_window"} | ({"nlm_pair"} if r else set())
     for e in entries:
         assert len(e["ms"]) == (2 if e["site"] == "nlm_window" else 3) and all(t >= 0 for t in e["ms"]), e
+
+
+def test_the_tuner_times_the_launches_a_frame_makes():
+    """A spatial pass's only window starts and finishes the frame, and a radius-1 pass's only pair starts
+    the sums: they are sites of their own, not those of passes with more windows."""
+    require_gpu()
+    W, H = 83, 47
+    geom = L.Geometry(W, H, 0, L.SampleFormat.u8(), L.SampleFormat.u8(), 0)
+    avd.set_tuning(True)
+    sites = {}
+    for r in (2, 1, 0):
+        opts = avd.nlmeans_options(temporal=1 if r else 0, temporal_radius=r, patch_radius=2, search_radius=2)
+        avd.build_engine("nlmeans", geom, luma=opts)
+        sites[r] = {(e["site"], e["key"]) for e in avd.tuning_entries() if f"{W}x{H}" in e["key"]}
+    assert {s for s, _ in sites[1] - sites[2]} == {"nlm_pair", "nlm_window"}
+    assert {s for s, _ in sites[0] - sites[1]} == {"nlm_single", "nlm_window"}
