@@ -886,7 +886,7 @@ __global__ __launch_bounds__(256) void k_centre_prep(const uint16_t *__restrict_
     __syncthreads();
     const int row = t / kRuns, run = t - row * kRuns;
     if (row >= kPrepRows || y0 + row > H - 8) return;
-    uint32_t e[kRun + 8];
+    __align__(16) uint32_t e[kRun + 8];
 #pragma unroll
     for (int i = 0; i < (kRun + 8) / 4; ++i) *(uint4 *)(e + 4 * i) = ((const uint4 *)&s_col[row][run * kRun])[i];
     uint32_t *to = energy + (size_t)(y0 + row) * W + x0 + run * kRun;

@@ -103,7 +103,7 @@ __global__ __launch_bounds__(kMeasureThreads) void k_grain_measure(
 {
     // The workgroup's counts gather in LDS and reach `hist` as one atomic per non-empty bin: a flat
     // region sends every cell to the same bin, where per-cell global atomics would serialise.
-    __shared__ int s_hist[2 * kHist];
+    __shared__ __align__(16) int s_hist[2 * kHist];  // cleared by 16-byte stores
     __shared__ int2 s_vec[kGroupY + 1][kGroupX + 2];  // the group's cells', the rim's cells' vectors
     __shared__ __align__(16) float s_grain[kPlaneH * kPlaneW];
     __shared__ __align__(16) float s_centre[kGroupY * kCell][kGroupX * kCell];  // mean-free
@@ -243,7 +243,7 @@ __global__ __launch_bounds__(kMeasureThreads) void k_grain_measure(
         const float *n_at = s_grain + (tcy * kCell + row) * kPlaneW + tcx * kCell + col;
 #pragma unroll 1
         for (int py = 0; py < kCell; ++py, c_at += kGroupX * kCell, n_at += kPlaneW) {
-            float c[kCell], n[kCell + kRun - 1];
+            __align__(16) float c[kCell], n[kCell + kRun - 1];
 #pragma unroll
             for (int i = 0; i < kCell / 4; ++i) *(float4 *)(c + 4 * i) = ((const float4 *)c_at)[i];
 #pragma unroll
