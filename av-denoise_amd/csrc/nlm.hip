@@ -63,6 +63,14 @@ struct Shape {
     static_assert(kWidth + 2 * P + 2 * kMaxS <= 64, "a tile row is staged by at most 64 lanes");
 };
 
+// Tile rows of a grid layer; taller frames take further layers along z, as a grid's y extent is limited to
+// 16 bits (three million frame rows at patch radius 8).  The last layer's surplus tiles write nothing.
+constexpr uint32_t kGridRows = 1u << 15;
+inline dim3 tile_grid(uint32_t columns, uint32_t rows)
+{
+    return dim3(columns, std::min(rows, kGridRows), div_up(rows, kGridRows));
+}
+
 // Samples between rows of a staged tile: odd, so that lanes on consecutive rows fall on distinct banks.
 __host__ __device__ inline int tile_pitch(int width, int P, int S) { return (width + 2 * P + 2 * S) | 1; }
 
@@ -302,7 +310,7 @@ __global__ __launch_bounds__(WX * SPLIT * 64) void k_nlm(NlmWindow w, const floa
     // Wave (wave, part): column run `wave` of the workgroup's WX, offset part `part` of SPLIT.
     const int lane = threadIdx.x & 63, id = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int wave = id % WX, part = id / WX;
-    const int X0 = blockIdx.x * T::kWidth, Y0 = blockIdx.y * T::kRows;
+    const int X0 = blockIdx.x * T::kWidth, Y0 = (int)(blockIdx.z * kGridRows + blockIdx.y) * T::kRows;
 
     // Tiles: columns X0-P-S .. X0+kWidth+P-1+S, rows Y0-P-S .. Y0+63-P+S.
     const int tcols = T::kWidth + 2 * P + 2 * S, trows = 64 + 2 * S, pitch = tile_pitch(T::kWidth, P, S);
@@ -366,7 +374,7 @@ __global__ __launch_bounds__(WX * SPLIT * 64) void k_nlm_window(NlmWindow w, Nlm
     const int S = w.S, W = w.W, H = w.H;
     const int lane = threadIdx.x & 63, id = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int wave = id % WX, part = id / WX;
-    const int X0 = blockIdx.x * T::kWidth, Y0 = blockIdx.y * T::kRows;
+    const int X0 = blockIdx.x * T::kWidth, Y0 = (int)(blockIdx.z * kGridRows + blockIdx.y) * T::kRows;
     const int tcols = T::kWidth + 2 * P + 2 * S, trows = 64 + 2 * S, pitch = tile_pitch(T::kWidth, P, S);
     const int tx0 = X0 - P - S, ty0 = Y0 - P - S;
     float *tf = lds;
@@ -487,7 +495,7 @@ hipError_t dispatch_split(const NlmWindow &w, const Window &a, bool pair, hipStr
 {
     constexpr int WS = waves_for(C, false, SPLIT), WP = waves_for(C, true, SPLIT);
     const size_t lds = tile_bytes(C, P, w.S, pair, COLS, SPLIT, pair ? WP : WS);
-    const dim3 grid(div_up(w.W, (pair ? WP : WS) * COLS), div_up(w.H, 64 - 2 * P));
+    const dim3 grid = tile_grid(div_up(w.W, (pair ? WP : WS) * COLS), div_up(w.H, 64 - 2 * P));
     auto launch = [&](auto kernel, int waves) {
         kernel<<<grid, waves * SPLIT * 64, lds, s>>>(w, a.centre, a.fwd, a.bwd, a.lut, a.conf_f, a.conf_b, a.accum,
                                                      a.wsum, a.maxw, a.fresh, a.self_weight, a.out);
@@ -539,7 +547,7 @@ hipError_t dispatch_window_split(const NlmWindow &w, const NlmFrames &f, const f
 {
     constexpr int WX = waves_for(C, true, SPLIT);
     const size_t lds = tile_bytes(C, P, w.S, f.pairs > 0, COLS, SPLIT, WX);
-    const dim3 grid(div_up(w.W, WX * COLS), div_up(w.H, 64 - 2 * P));
+    const dim3 grid = tile_grid(div_up(w.W, WX * COLS), div_up(w.H, 64 - 2 * P));
     const bool conf = f.pairs > 0 && f.conf_f[0] != nullptr;
     if (conf)
         k_nlm_window<C, P, COLS, WX, true, SPLIT><<<grid, WX * SPLIT * 64, lds, s>>>(w, f, centre, lut, self_weight,
