@@ -828,7 +828,8 @@ __global__ __launch_bounds__(kWaves * 64) void k_centre_codes(avd_collab_pass p,
 // (k_centre_redo).
 //
 // Bound by VALU issue: per key its distance and index (5 or 7 instructions) and the list's insertion
-// (KL), then the merge.  Alone, 3840x2160 with 16 members, one / two channels: with the codes in
+// (KL), then the merge.  One channel keeps four waves per SIMD at the price of seven spilled registers (write
+// traffic 110 MB at 3840x2160 with 16 members, whose words are 62).  Alone, 3840x2160 with 16 members, one / two channels: with the codes in
 // five-bit halves, a candidate row per product, its four operands loaded anew for each, and eight kept
 // keys per lane 1069 / 353 us, and 44 / 130 us of exact searches; this form 634 / 190 us, and 19 / 4 us.
 // ---------------------------------------------------------------------------------------------
@@ -1018,8 +1019,11 @@ __global__ __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_eu(C =
 
     // Each lane keeps its best KL keys per reference; a lane whose full list runs out during the merge
     // sends its reference to the exact search.
-    // Seven: with six a 427x241 frame
-    // of eight members sent a reference there (11 us for the one), an eighth costs a twentieth of the loop.
+    // Seven: a search of the list costs a reference's latency, 11 us, before it is work, and each kept key a
+    // part of the loop.  This kernel and the exact searches at six / seven / eight keys, one-channel planes,
+    // sums over three textured clips, us: 427x241 62 / 59 / 59, 640x360 79 / 71 / 74, 1280x720 208 / 196 / 201,
+    // 1920x1080 433 / 431 / 427 (eight members); 720x480 180 / 188 / 193, 1920x1080 709 / 672 / 688, 3840x2160
+    // 2589 / 2433 / 2484 (sixteen).
     constexpr int KL = 7;
     uint32_t L[2][KL];
 #pragma unroll

@@ -559,7 +559,8 @@ NlmWindow NlmPass::window() const
 
 // The window launch sites' columns per lane, picked by the tuner on this pass's own buffers, each launch as
 // denoise() makes it: ring slots, confidences and sums of hashed samples (see tuning_spread; the window walks
-// every offset whatever the content, so the time is the content's).  The stream then starts from scratch.
+// every offset whatever the content; flat content would only run the clock a few percent faster, for every
+// candidate).  The stream then starts from scratch.
 void NlmPass::tune_windows()
 {
     const size_t px = (size_t)W_ * H_;

@@ -23,11 +23,12 @@
 // shape.  On planes up to 2^20 pixels each tile's offsets are split over SPLIT waves whose sums add in
 // part order.  The sums leave through LDS, so global accumulators are read and written along rows.
 // Bound by vector instruction issue: per pixel and offset about 2 (1 + 2P / COLS) for the differences,
-// 4P + 1 for the box sums and 10 for the weight (v_exp_f32 issues over four cycles) and the sums.
-// Against lanes on columns (one pair or window of one frame, same sums): 640x360 P 2 S 7 81 -> 42 us,
-// 1920x1080 P 3 S 4 pair 541 -> 266 us, P 4 S 2 pair with confidence 276 -> 120 us, two-channel 960x540
-// P 3 S 4 pair 300 -> 113 us; the first runs at 85 % of its instruction issue bound (36 us at 240
-// workgroups on 256 CUs).
+// 4P + 1 for the box sums and 10 for the weight and the sums.  A wave's f32 add, subtract, multiply or
+// multiply-add issues in about 2.3 cycles, a max or a DPP add in four, v_exp_f32 in eight (measured): 62
+// cycles at P 2 and four columns, 77 at P 3.  Against lanes on columns (one pair or window of one frame,
+// same sums): 640x360 P 2 S 7 81 -> 42 us (22 of issue: two waves per SIMD leave latency in the open),
+// 1920x1080 P 3 S 4 pair 541 -> 266 us (185 of issue), P 4 S 2 pair with confidence 276 -> 120 us,
+// two-channel 960x540 P 3 S 4 pair 300 -> 113 us.
 // exp is v_exp_f32 (exp2) with log2(e) folded into h2 on the host.
 #include <algorithm>
 
